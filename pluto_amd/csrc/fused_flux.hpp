@@ -806,21 +806,30 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
 // z sweep, one thread per column marching over a z segment
 // ---------------------------------------------------------------------
 
+// A workgroup takes 256 consecutive columns of the plane, whatever the row
+// length, so only the plane's last workgroup has idle lanes (rows cut into
+// 64-wide tiles left 31% of the lanes of a 133-cell row idle: 133^3 171 ->
+// 121 us a launch, 131 x 93 x 77 81 -> 53).  At 256^3 the march moves its
+// 195 B per cell at 5.0 TB/s, the rate of a large copy; small boxes are
+// bound by the solves one after another along a segment (march_len).
+
 template <int STAGE, typename R, int S, int E, int V = 0>
-__global__ void __launch_bounds__(Z_TX * Z_TY)
+__global__ void __launch_bounds__(Z_COLS)
 k_flux_z(Geo g, StageIn in, Cons U, FaceData fd, const double* cdt_xy, int seg, DevScalars* sc)
 {
-  __shared__ double red[(Z_TX * Z_TY) / 64 + 1];
-  const int i = blockIdx.x * Z_TX + threadIdx.x;
-  const int j = blockIdx.y * Z_TY + threadIdx.y;
-  const ZSeg zs = zseg(g, blockIdx.z, seg);   // (a patch of a stack: z periodic within it)
+  __shared__ double red[Z_COLS / 64 + 1];
+  const unsigned col = blockIdx.x * (unsigned)Z_COLS + threadIdx.x;   // cell of the plane
+  // (its indices: only the reductions of a ghosted box ask for them)
+  const int j = g.ghost ? (int)(col / (unsigned)g.nx) : 0;
+  const int i = g.ghost ? (int)(col - (unsigned)j * (unsigned)g.nx) : 0;
+  const ZSeg zs = zseg(g, blockIdx.y, seg);   // (a patch of a stack: z periodic within it)
   const int k0 = zs.k0, k1 = zs.k1;
   sc = scal(sc, g, k0);
   double mach = 0.0, cdt_max = 0.0;
-  if (i < g.nx && j < g.ny) {
+  if (col < (unsigned)g.nx * (unsigned)g.ny) {
     // 32-bit byte offsets (the launcher keeps the z march to fields under
     // 4 GiB): the column's addresses stay one VGPR each
-    const unsigned col8 = ((unsigned)j * (unsigned)g.nx + (unsigned)i) * 8u;
+    const unsigned col8 = col * 8u;
     const unsigned pl8 = (unsigned)g.nx * (unsigned)g.ny * 8u;
     const double dt = sc->dt;
     const double dtdz = dt / g.dx[2];
@@ -995,15 +1004,13 @@ static void launch_flux_fused_t(const Geo& g, int stage, const StageIn& in, cons
   }
   if (kt) kt->end(KT_FLUX_XY, s);
   if (g.dims == 3) {
-    // z segment per column: 32 planes (one extra interface per segment),
-    // halved down to 16 while the box would get fewer than 512 workgroups
-    // (measured: 256^3 best at 32, 128^3 at 16)
-    const long xy = (long)((g.nx + Z_TX - 1) / Z_TX) * ((g.ny + Z_TY - 1) / Z_TY);
-    const int pz = patch_depth(g);
-    int seg = pz >= 64 ? 32 : (pz >= 16 ? 8 : pz);
-    if (seg == 32 && xy * zblocks(g, seg) < 512) seg = 16;
-    const dim3 bz(Z_TX, Z_TY), gz((g.nx + Z_TX - 1) / Z_TX, (g.ny + Z_TY - 1) / Z_TY,
-                                  zblocks(g, seg));
+    const unsigned cols = (unsigned)g.nx * (unsigned)g.ny, wgs = (cols + Z_COLS - 1) / Z_COLS;
+    // (the FP32 z march is memory-bound and best on short segments: 256^3
+    // 518 us at 8 planes, 534 at 32)
+    const int seg = march_len(sizeof(R) == 4 ? 8 : 32, patch_depth(g), [&](int len) {
+      return (long)wgs * (Z_COLS / 64) * zblocks(g, len);
+    });
+    const dim3 bz(Z_COLS), gz(wgs, zblocks(g, seg));
     if (kt) kt->begin(KT_FLUX_Z, s);
     if (stage == 1)
       hipLaunchKernelGGL((k_flux_z<1, R, S, E, V>), gz, bz, 0, s, g, in, U, fd, cdt_xy, seg, sc);

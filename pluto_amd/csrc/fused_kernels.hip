@@ -129,10 +129,10 @@ __global__ void __launch_bounds__(256) k_ct_c2p_z(Geo g, EdgeOut e, FaceIn bin, 
                                                   FaceOut bout, Cons U, StageIn vn, Prims Vout,
                                                   unsigned char* flag, DevScalars* sc, int kz)
 {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = blockIdx.y * blockDim.y + threadIdx.y;
-  if (i >= g.nx || j >= g.ny) return;
-  const ZSeg zs = zseg(g, blockIdx.z, kz);   // (a patch of a stack: z periodic within it)
+  const unsigned col = blockIdx.x * blockDim.x + threadIdx.x;   // cell of the plane
+  if (col >= (unsigned)g.nx * (unsigned)g.ny) return;
+  const int j = (int)(col / (unsigned)g.nx), i = (int)(col - (unsigned)j * (unsigned)g.nx);
+  const ZSeg zs = zseg(g, blockIdx.y, kz);   // (a patch of a stack: z periodic within it)
   sc = scal(sc, g, zs.k0);
   const double dt = sc->dt;
   const double dtx = dt / g.dx[0], dty = dt / g.dx[1], dtz = dt / g.dx[2];
@@ -229,25 +229,25 @@ int launch_ct_c2p(const Geo& g, int stage, const EdgeOut& e, const FaceIn& bin, 
   if (f32_out && stage != 1) return (int)hipErrorInvalidValue;
   const bool zmarch = g.dims == 3 && (unsigned long long)g.n * 8ull < (1ull << 32);
   if (g.pz > 0 && !zmarch) return (int)hipErrorInvalidValue;   // stacks: the z march only
-  // rows of 128 cells x 2 (less y halo re-read than 64 x 4: 0.81 -> 0.78 ms
-  // at 256^3) where that wastes no more lanes than 64 x 4 (261-cell rows of
-  // a ghosted box: 64 x 4)
-  const int bx = (g.nx + 127) / 128 * 128 <= (g.nx + 63) / 64 * 64 ? 128 : 64, by = 256 / bx;
-  const dim3 b(bx, by), gr((g.nx + bx - 1) / bx, (g.ny + by - 1) / by, g.nz);
+  const dim3 b(64, 4), gr((g.nx + 63) / 64, (g.ny + 3) / 4, g.nz);
   if (kt) kt->begin(KT_CT, s);
   if (zmarch) {
     // planes per workgroup: up to 16, fewer while the box would get fewer
     // than 2048 workgroups
-    const long xy = (long)gr.x * gr.y;
+    const unsigned cols = (unsigned)g.nx * (unsigned)g.ny;
+    // 256 consecutive columns of the plane per workgroup, whatever the row
+    // length: 133^3 135 -> 104 us a launch, 131 x 93 x 77 58 -> 44 (64 x 4
+    // tiles leave lanes idle at the row ends); 128 and 64 columns: 112, 117
+    const unsigned wgs = (cols + 255) / 256;
     int kz = 16;
-    while (kz > 1 && xy * zblocks(g, kz) < 2048) kz /= 2;
-    const dim3 gz(gr.x, gr.y, zblocks(g, kz));
+    while (kz > 1 && (long)wgs * zblocks(g, kz) < 2048) kz /= 2;
+    const dim3 gz(wgs, zblocks(g, kz)), bz(256);
     if (f32_out)
-      hipLaunchKernelGGL((k_ct_c2p_z<1, true>), gz, b, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, kz);
+      hipLaunchKernelGGL((k_ct_c2p_z<1, true>), gz, bz, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, kz);
     else if (stage == 1)
-      hipLaunchKernelGGL((k_ct_c2p_z<1, false>), gz, b, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, kz);
+      hipLaunchKernelGGL((k_ct_c2p_z<1, false>), gz, bz, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, kz);
     else
-      hipLaunchKernelGGL((k_ct_c2p_z<2, false>), gz, b, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, kz);
+      hipLaunchKernelGGL((k_ct_c2p_z<2, false>), gz, bz, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, kz);
   } else if (f32_out) {
     hipLaunchKernelGGL((k_ct_c2p<1, true>), gr, b, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc);
   } else if (stage == 1) {

@@ -6,7 +6,34 @@
 namespace pgpu {
 
 constexpr int XY_TX = 32, XY_TY = 8;   // k_flux_xy workgroup (one z-plane); FP64 tiles overlap
-constexpr int Z_TX = 64, Z_TY = 4;     // k_flux_z columns per workgroup
+constexpr int Z_COLS = 256;            // k_flux_z columns per workgroup, consecutive in the plane
+
+// Cells of a march's segment (a power of two up to `most`, no longer than the
+// line needs) for kernels that solve Riemann problems one after another
+// along it at two waves per SIMD; waves(len): waves of the launch.  A wave
+// does len + 2 interfaces' work (one solved again and two reconstructions
+// at the segment's start), the 1024 SIMDs take up to 2048 waves at a time,
+// and a round with two waves per SIMD takes 1.5 times one with a single
+// wave (measured).  The estimate orders the measured times right: z march
+// of 64^3 seg 4: 26 us (8: 32, 16: 50), 96^3 8: 51 (16: 57, 4: 58), 128^3 16: 93
+// (8: 100, 32: 113), 133^3 8: 121 (16: 132, 4: 133), 384 x 288 x 320 32: 1414
+// (16: 1448, 64: 1465), 32^3 1: 13 (8: 30).
+template <class W>
+inline int march_len(int most, int line, W waves)
+{
+  int best = 1;
+  double cost = 0.0;
+  for (int len = 1; len <= most && (len == 1 || len < 2 * line); len *= 2) {
+    const long w = waves(len), rest = w % 2048;
+    const double rounds = 1.5 * (double)(w / 2048) + (rest > 1024 ? 1.5 : (rest > 0 ? 1.0 : 0.0));
+    const double c = rounds * (len + 2);
+    if (len == 1 || c <= cost) {
+      best = len;
+      cost = c;
+    }
+  }
+  return best;
+}
 
 // Per-face UCT_HLL speeds and per-cell velocity slopes written by the flux
 // kernels for the EMF kernel (same arrays as SweepOut's).

@@ -1,0 +1,60 @@
+"""Boxes at the edges of the launch shapes against the oracle, bit for bit."""
+import pytest
+
+from conftest import assert_states_equal
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def box_state(shape, dims=3, seed=11):
+    """A seeded state on a box of any shape: periodic plane waves."""
+    import numpy as np
+
+    from pluto_amd import problems as P
+    rng = np.random.default_rng([seed, dims, *shape])
+    nz, ny, nx = shape
+    d = (1.0 / nx, 1.0 / ny, 1.0 / nz if dims == 3 else 1.0)
+
+    def field():
+        f = np.zeros(shape)
+        for _ in range(6):
+            k = rng.integers(-3, 4, 3)
+            a = [2 * np.pi * k[c] * (np.arange(n) + 0.5) / n for c, n in enumerate((nx, ny, nz))]
+            f += rng.standard_normal() * np.cos(a[0][None, None, :] + a[1][None, :, None]
+                                                + a[2][:, None, None] * (dims == 3)
+                                                + rng.uniform(0, 6.28))
+        return f / 6.0
+
+    a = [0.05 * field() for _ in range(3)]
+    if dims == 2:
+        a[0][:], a[1][:] = 0.0, 0.0
+    b = P.curl_edges(*a, d, dims)
+    v = np.stack([0.4 * field() for _ in range(3)])
+    if dims == 2:
+        v[2] = 0.0
+    return P.assemble(1.0 + 0.3 * field(), v, 1.0 + 0.3 * field(), *b, dims, (1.0, 1.0, 1.0))
+
+
+def check(shape, steps=2, dims=3, **kw):
+    from pluto_amd import native
+    st = box_state(shape, dims)
+    dt = 0.05 / max(shape)
+    dom = native.Domain.from_state(st, **kw)
+    dom.set_dt(dt)
+    dom.run(steps)
+    dom.sync()
+    out = dom.get_state(st)
+    dom.close()
+    ref = st.copy()
+    O.run(ref, steps, dt)
+    assert_states_equal(out, ref, "%s" % (shape,))
+
+
+# the z march and the CT march: 256 columns of the plane per workgroup (255,
+# 256, 257 columns), segments of 1 plane and longer ones with a remainder (by
+# size: 2, 4, 8 and 32 planes)
+@pytest.mark.parametrize("shape", [(3, 17, 15), (5, 16, 16), (4, 257, 3), (7, 4, 64), (49, 48, 47),
+                                   (65, 64, 63), (77, 93, 131), (161, 160, 160)])
+def test_marches(shape):
+    check(shape)
