@@ -477,11 +477,22 @@ k_flux_xy_items(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScala
 constexpr int XROW_NV = NV - 1;
 __device__ __forceinline__ constexpr int xrow_var(int q) { return q < BX1 ? q : q + 1; }
 
-// The workgroup holds one whole box row (thread i = cell i, nx <= MAXT,
-// nx even) of plane k and marches up the rows j0 .. j0+seg-1.  Rows of the
-// primitive state go through a ring of three LDS row buffers, filled by
-// direct global-to-LDS copies (global_load_lds_dwordx4, no registers on
-// the way) one row ahead.  For row j each thread
+// A workgroup takes up to MAXT cells along x and marches up the rows
+// j0 .. j0+seg-1 of their planes.  How its threads sit on the box (RowMap)
+// is a launch parameter:
+//   rows > 0   thread t = cell t % nx of plane blockIdx.y * rows + t / nx:
+//              whole rows of `rows` planes, each periodic within itself
+//   rows = 0   the rows of all planes, each with the images of its last two
+//              cells before it and of its first two after it (nx + 4 threads),
+//              one after another; workgroup w takes the window of blockDim.x
+//              threads that starts at w * (blockDim.x - 4).  The window's
+//              two outer threads at either end and the images only feed their
+//              neighbours: any row length, about 1 - 4/256 - 4/nx of the lanes
+//              busy
+// Rows of the primitive state go through a ring of three LDS row buffers,
+// filled by direct global-to-LDS copies (global_load_lds_dword, no registers
+// on the way, any alignment) one row ahead, every wave its own 64 cells.
+// For row j each thread
 //   - reconstructs its own cell in x (PLM from the ring, periodic
 //     neighbours), solves the x interface i-1/2 with its left neighbour's
 //     right-face state from LDS, and takes the flux at i+1/2 from its right
@@ -499,14 +510,51 @@ __device__ __forceinline__ constexpr int xrow_var(int q) { return q < BX1 ? q : 
 // so the results are identical.
 // LDS (dynamic): 3 * NV * blockDim.x ring values and (NV + 7) * blockDim.x
 // values of R.
+
+// thread t of workgroup w: its cell (ic, k), whether it owns that cell's
+// results, and the threads of its x neighbours
+struct RowCell {
+  int ic, k, tl, tr;
+  bool act;
+};
+
+__device__ __forceinline__ RowCell row_cell(const Geo& g, int rows, int w, int t, int nt)
+{
+  RowCell c;
+  if (rows > 0) {
+    int r = t / g.nx;
+    c.act = r < rows && w * rows + r < g.nz;
+    r = min(r, rows - 1);
+    c.ic = t - r * g.nx;
+    c.k = min(w * rows + r, g.nz - 1);
+    c.tl = c.ic == 0 ? t + g.nx - 1 : t - 1;
+    c.tr = c.ic == g.nx - 1 ? t - (g.nx - 1) : t + 1;
+    if (c.ic >= g.nx) {   // past the last row
+      c.ic = g.nx - 1;
+      c.tl = c.tr = t;
+    }
+  } else {
+    const int f = w * (nt - 4) + t, len = g.nx + 4;
+    c.k = f / len;
+    const int q = f - c.k * len - 2;   // -2, -1: images of the last cells, nx, nx + 1: of the first
+    c.act = t > 1 && t < nt - 2 && q >= 0 && q < g.nx && c.k < g.nz;
+    c.ic = q < 0 ? q + g.nx : (q >= g.nx ? q - g.nx : q);
+    c.k = min(c.k, g.nz - 1);
+    c.tl = max(t - 1, 0);
+    c.tr = min(t + 1, nt - 1);
+  }
+  return c;
+}
+
 template <int STAGE, typename R, int S, int E, int V, int MAXT>
 __global__ void __launch_bounds__(MAXT, 2)
-k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, DevScalars* sc)
+k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, int rows,
+               DevScalars* sc)
 {
   // rows of the state as they are stored: FP64, or float for the FP32-flux
-  // path's second stage; CPL cells per 16-byte lane copy
+  // path's second stage; a lane copies 4 bytes, CPC lanes a cell
   using RT = std::conditional_t<(STAGE == 2 && sizeof(R) == 4), float, double>;
-  constexpr int CPL = 16 / int(sizeof(RT)), CCH = 64 * CPL;
+  constexpr int CPC = int(sizeof(RT)) / 4, CCH = 64 / CPC;   // cells per copy
   extern __shared__ __align__(16) unsigned char xrow_lds[];
   __shared__ double red[MAXT / 64 + 1];
   const int nt = blockDim.x;
@@ -514,30 +562,30 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
   R* xp = reinterpret_cast<R*>(ring + 3 * NV * nt);   // [NV][nt] right-face states, B_x: the face value
   R* xf = xp + NV * nt;                               // [7][nt] flux at i-1/2: rho mx my mz E p cmax
 
-  const int i = threadIdx.x;
-  const int lane = i & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(i >> 6);
-  const int nwave = nt >> 6;
-  const bool act = i < g.nx;
-  const int ic = act ? i : g.nx - 1;
-  const int il = ic == 0 ? g.nx - 1 : ic - 1;
-  const int ir = ic == g.nx - 1 ? 0 : ic + 1;
+  const int t = threadIdx.x;
+  const int lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const dim3 tb = xcd_tile();
-  const int j0 = tb.x * seg, k = tb.y;
+  const int j0 = tb.x * seg;
   const int j1 = min(j0 + seg, g.ny);
-  sc = scal(sc, g, k);
+  const RowCell rc = row_cell(g, rows, tb.y, t, nt);
+  const bool act = rc.act;
+  const int ic = rc.ic, k = rc.k, tl = rc.tl, tr = rc.tr;
+  sc = scal(sc, g, (int)tb.y * rows);   // (a stack: the workgroup's rows are of one patch)
   // 32-bit byte offsets of FP64 fields (the launcher keeps this kernel to
   // boxes under 4 GiB per field): the loop's addresses stay one VGPR each
-  const unsigned plane8 = (unsigned)k * (unsigned)g.ny * (unsigned)g.nx * 8u;
   const unsigned row8 = (unsigned)g.nx * 8u;
+  const unsigned plane8 = row8 * (unsigned)g.ny;
+  const unsigned col8 = (unsigned)k * plane8 + (unsigned)ic * 8u;    // cell (ic, 0, k)
+  const unsigned coll8 = col8 - (ic == 0 ? 0u - (row8 - 8u) : 8u);   // its left neighbour
   const double dt = sc->dt;
   const double dtdx = dt / g.dx[0], dtdy = dt / g.dx[1];
   const R gam = R(g.gamma), gm1 = R(g.gmm1);
   double mach = 0.0;
 
-  auto off8 = [&](int jj, int ii) { return plane8 + (unsigned)jj * row8 + (unsigned)ii * 8u; };
+  auto off8 = [&](int jj) { return col8 + (unsigned)jj * row8; };
   auto load = [&](int jj, R* v) {
-    const unsigned o = off8(wrap_any(jj, g.ny), ic);
+    const unsigned o = off8(wrap_any(jj, g.ny));
 #pragma unroll
     for (int q = 0; q < NV; q++)
       v[q] = sizeof(RT) == 4 ? R(at_byte(reinterpret_cast<const float*>(in.V[q]), o >> 1))
@@ -548,19 +596,25 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
     if constexpr (sizeof(R) == 4) at_byte(reinterpret_cast<float*>(a), o >> 1) = v;
     else at_byte(a, o) = v;
   };
-  // copy row jj of every variable into ring slot sl: 16 bytes (CPL cells)
-  // per lane, chunks of CCH cells dealt to the waves in turn
-  const int nchunk = (g.nx + CCH - 1) / CCH;
+  // copy row jj of every variable into ring slot sl: each wave the cells of
+  // its own threads, CCH of them per copy
+  unsigned soff[CPC];
+#pragma unroll
+  for (int c = 0; c < CPC; c++) {
+    const RowCell s = row_cell(g, rows, tb.y, wave * 64 + c * CCH + lane / CPC, nt);
+    soff[c] = ((unsigned)s.k * plane8 + (unsigned)s.ic * 8u) / (8u / sizeof(RT)) +
+              (unsigned)(lane % CPC) * 4u;
+  }
   auto stage_row = [&](int jj, int sl) {
-    const unsigned o = off8(wrap_any(jj, g.ny), 0) / (8u / sizeof(RT));   // byte offset of the row
-    for (int n = wave; n < NV * nchunk; n += nwave) {
-      const int q = n / nchunk, c = n - q * nchunk;
-      const int cell = c * CCH + CPL * lane;
-      if (cell < g.nx)
+    const unsigned o = (unsigned)wrap_any(jj, g.ny) * (row8 / (8u / (unsigned)sizeof(RT)));
+#pragma unroll
+    for (int q = 0; q < NV; q++)
+#pragma unroll
+      for (int c = 0; c < CPC; c++)
         __builtin_amdgcn_global_load_lds(
-            (const void*)(reinterpret_cast<const char*>(in.V[q]) + (o + (unsigned)cell * (unsigned)sizeof(RT))),
-            (__attribute__((address_space(3))) void*)(ring + (sl * NV + q) * nt + c * CCH), 16, 0, 0);
-    }
+            (const void*)(reinterpret_cast<const char*>(in.V[q]) + (o + soff[c])),
+            (__attribute__((address_space(3))) void*)(ring + (sl * NV + q) * nt + wave * 64 + c * CCH),
+            4, 0, 0);
   };
   // wait for every vector memory access of this thread (the ring copies
   // among them) before a barrier that publishes the copies
@@ -569,7 +623,7 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
   // velocity slopes of the y reconstruction of cell (i, jj)
   auto store_dvy = [&](int jj, const R* vp, const R* vm) {
     if constexpr (E != FACE_BFLUX) {
-      const unsigned o = off8(jj, ic);
+      const unsigned o = off8(jj);
       fstore(fd.dv[1][0], o, vp[VX1] - vm[VX1]);
       fstore(fd.dv[1][1], o, vp[VX2] - vm[VX2]);
       fstore(fd.dv[1][2], o, vp[VX3] - vm[VX3]);
@@ -595,7 +649,7 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
       vL[q] = vpb[q];
       vR[q] = vm0[q];
     }
-    const R bface = R(at_byte(in.b[1], off8(wrap_any(j0 - 1, g.ny), ic)));
+    const R bface = R(at_byte(in.b[1], off8(wrap_any(j0 - 1, g.ny))));
     vL[BX2] = bface;
     vR[BX2] = bface;
     RiemannOut<R> r;
@@ -616,13 +670,13 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
   constexpr bool kPrefetch = sizeof(R) == sizeof(double);
   R bfx_n = R(0), bfy_n = R(0);
   if (kPrefetch) {
-    bfx_n = R(at_byte(in.b[0], off8(j0, il)));
-    bfy_n = R(at_byte(in.b[1], off8(j0, ic)));
+    bfx_n = R(at_byte(in.b[0], coll8 + (unsigned)j0 * row8));
+    bfy_n = R(at_byte(in.b[1], off8(j0)));
   }
   int s0 = 0, s1 = 1, s2 = 2;   // ring slots of rows j, j+1, j+2
   for (int j = j0; j < j1; j++) {
-    const unsigned c = off8(j, ic);
-    const unsigned cf = off8(j, il);   // owner cell of the x face i-1/2
+    const unsigned c = off8(j);
+    const unsigned cf = coll8 + (unsigned)j * row8;   // owner cell of the x face i-1/2
     const R bfx = kPrefetch ? bfx_n : R(at_byte(in.b[0], cf));
     const R bfy = kPrefetch ? bfy_n : R(at_byte(in.b[1], c));
 
@@ -632,11 +686,11 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
     {
       R w0[NV], a[NV], b[NV], vpx[NV];
 #pragma unroll
-      for (int q = 0; q < NV; q++) w0[q] = rv(s0, q, ic);
+      for (int q = 0; q < NV; q++) w0[q] = rv(s0, q, t);
       if (STAGE == 1) {   // U0 from the FP64 state
         double v[NV];
 #pragma unroll
-        for (int q = 0; q < NV; q++) v[q] = double(ring[(s0 * NV + q) * nt + ic]);
+        for (int q = 0; q < NV; q++) v[q] = double(ring[(s0 * NV + q) * nt + t]);
         u[0] = v[RHO];
         u[1] = v[RHO] * v[VX1];
         u[2] = v[RHO] * v[VX2];
@@ -645,8 +699,8 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
       }
 #pragma unroll
       for (int q = 0; q < XROW_NV; q++) {
-        a[xrow_var(q)] = rv(s0, xrow_var(q), il);
-        b[xrow_var(q)] = rv(s0, xrow_var(q), ir);
+        a[xrow_var(q)] = rv(s0, xrow_var(q), tl);
+        b[xrow_var(q)] = rv(s0, xrow_var(q), tr);
       }
       a[BX1] = w0[BX1];   // not used: the x interfaces take the face value
       b[BX1] = w0[BX1];
@@ -654,7 +708,7 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
       // (every thread writes its slot: the face value's load then stays
       // at the top of the row instead of sinking into a branch)
 #pragma unroll
-      for (int q = 0; q < NV; q++) xp[q * nt + i] = q == BX1 ? bfx : vpx[q];
+      for (int q = 0; q < NV; q++) xp[q * nt + t] = q == BX1 ? bfx : vpx[q];
       if (act) {
         if constexpr (E != FACE_BFLUX) {
           fstore(fd.dv[0][0], c, vpx[VX1] - vmx[VX1]);
@@ -668,8 +722,8 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
     if (j + 1 < j1) {
       stage_row(j + 2, s2);
       if (kPrefetch) {
-        bfx_n = R(at_byte(in.b[0], off8(j + 1, il)));
-        bfy_n = R(at_byte(in.b[1], off8(j + 1, ic)));
+        bfx_n = R(at_byte(in.b[0], coll8 + (unsigned)(j + 1) * row8));
+        bfy_n = R(at_byte(in.b[1], off8(j + 1)));
       }
     }
 
@@ -678,10 +732,10 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
     {
       R vL[NV], vR[NV];
 #pragma unroll
-      for (int q = 0; q < NV; q++) vL[q] = xp[q * nt + il];
+      for (int q = 0; q < NV; q++) vL[q] = xp[q * nt + tl];
 #pragma unroll
       for (int q = 0; q < NV; q++) vR[q] = vmx[q];
-      const R bface = xp[BX1 * nt + i];
+      const R bface = xp[BX1 * nt + t];
       vL[BX1] = bface;
       vR[BX1] = bface;
       RiemannOut<R> r;
@@ -697,10 +751,10 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
         xsl = max_ge(R(0), -r.SL);
         xsr = max_ge(R(0), r.SR);
       }
-      if (act) {
 #pragma unroll
-        for (int q = 0; q < 6; q++) xf[q * nt + i] = fxl[q];
-        xf[6 * nt + i] = cmxl;
+      for (int q = 0; q < 6; q++) xf[q * nt + t] = fxl[q];
+      xf[6 * nt + t] = cmxl;
+      if (act) {
         const double rm = double(r.mach);
         if (in_sweep(g, 0, ic - 1, j, k)) mach = rm > mach ? rm : mach;
       }
@@ -724,9 +778,9 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
     }
     double rx[5], cdt = 0.0;
 #pragma unroll
-    for (int q = 0; q < 5; q++) rx[q] = -dtdx * (double(xf[q * nt + ir]) - double(fxl[q]));
-    rx[1] -= dtdx * (double(xf[5 * nt + ir]) - double(fxl[5]));
-    if (STAGE == 1) cdt += 0.5 * (double(cmxl) + double(xf[6 * nt + ir])) * g.inv_dx[0];
+    for (int q = 0; q < 5; q++) rx[q] = -dtdx * (double(xf[q * nt + tr]) - double(fxl[q]));
+    rx[1] -= dtdx * (double(xf[5 * nt + tr]) - double(fxl[5]));
+    if (STAGE == 1) cdt += 0.5 * (double(cmxl) + double(xf[6 * nt + tr])) * g.inv_dx[0];
 
     // y reconstruction of cell (i, j+1) and the y interface j+1/2
     R vpn[NV], vmn[NV];
@@ -734,12 +788,12 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
       R a[NV], b[NV], w2[NV];
 #pragma unroll
       for (int q = 0; q < NV; q++) {
-        a[q] = rv(s0, q, ic);
-        b[q] = rv(s1, q, ic);
+        a[q] = rv(s0, q, t);
+        b[q] = rv(s1, q, t);
       }
       if (j + 1 < j1) {
 #pragma unroll
-        for (int q = 0; q < NV; q++) w2[q] = rv(s2, q, ic);
+        for (int q = 0; q < NV; q++) w2[q] = rv(s2, q, t);
       } else {
         load(j + 2, w2);   // the segment's last row: row j+2 is not staged
       }
@@ -972,22 +1026,17 @@ static void launch_flux_fused_t(const Geo& g, int stage, const StageIn& in, cons
   if (kt) kt->begin(KT_FLUX_XY, s);
   bool rows = false;
   {
-    // the row kernel: rows of up to 256 cells, an even number (FP64) or a
-    // multiple of 4 (FP32 flux: the second stage's float rows), fields under
-    // 4 GiB (Roe's FP64 row kernel spills about 50 VGPRs and still beats the
-    // tiles: 2.37 -> 2.07 ms at 256^3)
-    const int nt = (g.nx + 63) / 64 * 64;
-    rows = flux_rows_ok(g, (int)sizeof(R), S);
+    const RowLaunch rl = row_launch(g, (int)sizeof(R));
+    rows = rl.nt > 0;
     if (rows) {
-      const int seg = flux_xy_seg(g);
-      const dim3 grid((g.ny + seg - 1) / seg, g.nz), block(nt);
+      const dim3 grid((g.ny + rl.seg - 1) / rl.seg, rl.wgs), block(rl.nt);
       // ring rows: FP64, except the FP32-flux path's float second-stage input
       const size_t rt = (stage == 2 && sizeof(R) == 4) ? 4 : 8;
-      const size_t lds = 3 * NV * nt * rt + (NV + 7) * nt * sizeof(R);
+      const size_t lds = 3 * NV * rl.nt * rt + (NV + 7) * rl.nt * sizeof(R);
       if (stage == 1)
-        hipLaunchKernelGGL((k_flux_xy_rows<1, R, S, E, V, 256>), grid, block, lds, s, g, in, U, fd, cdt_xy, seg, sc);
+        hipLaunchKernelGGL((k_flux_xy_rows<1, R, S, E, V, 256>), grid, block, lds, s, g, in, U, fd, cdt_xy, rl.seg, rl.rows, sc);
       else
-        hipLaunchKernelGGL((k_flux_xy_rows<2, R, S, E, V, 256>), grid, block, lds, s, g, in, U, fd, cdt_xy, seg, sc);
+        hipLaunchKernelGGL((k_flux_xy_rows<2, R, S, E, V, 256>), grid, block, lds, s, g, in, U, fd, cdt_xy, rl.seg, rl.rows, sc);
     }
   }
   if (rows) {

@@ -271,16 +271,7 @@ int set_flux_xy_kernel(int kind, int seg)
 
 int flux_xy_kind() { return g_flux_xy_kind; }
 
-int flux_xy_seg(const Geo& g)
-{
-  if (g_flux_xy_seg > 0) return g_flux_xy_seg;
-  // 32 rows, halved (down to 4) while the box would get fewer than 2048
-  // waves (8 per CU); measured: 256^3 best at 32 (8192 waves), 128^3 at 16
-  const long waves_per_row = (g.nx + 63) / 64;
-  int seg = 32;
-  while (seg > 4 && (long)((g.ny + seg - 1) / seg) * g.nz * waves_per_row < 2048) seg /= 2;
-  return seg;
-}
+int flux_xy_seg() { return g_flux_xy_seg; }
 
 int launch_flux_fused(const Geo& g, int stage, bool fp32_flux, const StageIn& in, const Cons& U,
                       const FaceData& fd, double* cdt_xy, DevScalars* sc, hipStream_t s,
@@ -288,7 +279,7 @@ int launch_flux_fused(const Geo& g, int stage, bool fp32_flux, const StageIn& in
 {
   // a stack of patches runs on the row kernel (its z march handles stacks);
   // the z march takes 32-bit offsets: 3D fields under 4 GiB
-  if (g.pz > 0 && (g.dims != 3 || !flux_rows_ok(g, fp32_flux ? 4 : 8, g.solver)))
+  if (g.pz > 0 && (g.dims != 3 || !row_launch(g, fp32_flux ? 4 : 8).nt))
     return (int)hipErrorInvalidValue;
   if (g.dims == 3 && g.n * 8 >= (1l << 32)) return (int)hipErrorInvalidValue;
   if (g.emf_avg != EMF_UCT_HLL) {

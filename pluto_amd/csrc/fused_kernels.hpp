@@ -57,21 +57,65 @@ int launch_flux_fused_fast(const Geo& g, int stage, const StageIn& in, const Con
                            KernelTimer* kt);
 // x/y flux kernel of the fused stage (process-wide; FP64 results identical,
 // FP32-flux ones to FP32 rounding: the two kernels contract differently):
-// 0 the overlapping z-plane tiles (k_flux_xy, k_flux_xy_items), 1 whole
-// rows marching up y segments of seg rows (k_flux_xy_rows; 0: by the box's
-// size, flux_xy_seg) on boxes with nx even (FP32 flux: a multiple of 4),
-// 4 <= nx <= 256, ny >= 4 and fields under 4 GiB; the tiles elsewhere
+// 0 the overlapping z-plane tiles (k_flux_xy, k_flux_xy_items), 1 rows
+// marching up y segments of seg rows (k_flux_xy_rows; 0: by the box's size,
+// and the FP64 tiles on boxes so small that they take less time)
 int set_flux_xy_kernel(int kind, int seg);
 int flux_xy_kind();
-int flux_xy_seg(const Geo& g);
-// the row kernel takes this box (flux real type of real_bytes, solver)
-inline bool flux_rows_ok(const Geo& g, int real_bytes, int solver)
+int flux_xy_seg();
+
+// Launch shape of the row kernel: nt threads, wgs workgroups across the
+// planes (nt = 0: this box takes the tiles), rows per workgroup (0: windows)
+// and rows of a y segment, the combination with the least estimated time.
+// In units of a row of two-waves-per-SIMD work (9.6 us): a workgroup takes
+// len + 1.3 of them (an interface and two reconstructions more at a
+// segment's start), 512 workgroups of three or four waves (three: 0.8 of
+// the time) run at once, half as many in 0.65 of the time; whole rows go in
+// rounds, the windows' workgroups drift apart and end ragged (f + 0.4).
+// Measured at 256^3 1255 us (16 rows: 1294), 128^3 as two rows a workgroup
+// 176 (one row: 180, and 299 against 206 at 32 rows), 64^3 36 (one row a
+// workgroup: 47), 16 x 256^2 91 (windows of one row: 196), 133^3 windows
+// 8 rows 278 (32: 304), 261 x 256^2 16 rows 1345 (8: 1434), 384 x 288 x 320
+// 2790 (tiles: 3792).
+struct RowLaunch {
+  int nt = 0, wgs = 0, rows = 0, seg = 0;
+};
+
+inline RowLaunch row_launch(const Geo& g, int real_bytes)
 {
-  const int nt = (g.nx + 63) / 64 * 64;
-  (void)solver;
-  return flux_xy_kind() == 1 && g.nx >= 4 &&
-         g.nx % (real_bytes == 4 ? 4 : 2) == 0 && nt <= 256 && g.ny >= 4 &&
-         g.n * 8 < (1l << 32);
+  RowLaunch best;
+  if (flux_xy_kind() != 1 || g.n * 8 >= (1l << 32)) return best;
+  double cost = 0.0;
+  auto offer = [&](int nt, long wgs, int rows) {
+    const int lens = flux_xy_seg() > 0 ? flux_xy_seg() : 32;
+    for (int len = flux_xy_seg() > 0 ? lens : 1; len <= lens && (len <= g.ny || lens == len); len++) {
+      const double f = (double)(wgs * ((g.ny + len - 1) / len)) * (nt <= 128 ? nt / 256.0 : 1.0) / 512.0;
+      const double all = rows > 0 ? (f <= 4.0 ? (double)(long)(f + 0.9999) : f)
+                                  : (f <= 0.75 ? 1.0 : f + 0.4);
+      const double c = (f <= 0.5 ? 0.65 : all) * (len + 1.3) * (nt == 192 ? 0.8 : (nt < 192 ? 1.1 : 1.0));
+      if (best.nt && c > cost) continue;
+      best.nt = nt;
+      best.wgs = (int)wgs;
+      best.rows = rows;
+      best.seg = len;
+      cost = c;
+    }
+  };
+  const int deep = patch_depth(g);
+  // (a workgroup's rows belong to one patch of a stack, which has no windows)
+  if (g.pz <= 0)
+    for (int nt = 64; nt <= 256; nt += 64)
+      offer(nt, ((long)g.nz * (g.nx + 4) - 4 + nt - 5) / (nt - 4), 0);
+  for (int r = 1; r * g.nx <= 256 && r <= deep; r++)
+    if (g.pz <= 0 || deep % r == 0) offer((r * g.nx + 63) / 64 * 64, ((long)g.nz + r - 1) / r, r);
+  if (real_bytes == 8 && g.pz <= 0 && flux_xy_seg() <= 0) {
+    // the tiles: 768 workgroups at once, 17 us a round (48^3: 26 us, rows 30;
+    // a 512^2 plane 37, rows 48; 64^3: 51, rows 36)
+    const double f = (double)((g.nx + 30) / 31) * ((g.ny + 6) / 7) * g.nz / 768.0;
+    const double us = f <= 1.0 ? 12.0 + 14.0 * f : 3.0 + 17.0 * (f <= 4.0 ? (double)(long)(f + 0.9999) : f + 0.3);
+    if (us < 5.0 + 9.6 * cost) best.nt = 0;
+  }
+  return best;
 }
 // the FP32-flux launches (fused_f32.hip, compiled with FMA contraction)
 int launch_flux_fused_f32(const Geo& g, int stage, const StageIn& in, const Cons& U,

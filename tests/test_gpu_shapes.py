@@ -58,3 +58,19 @@ def check(shape, steps=2, dims=3, **kw):
                                    (65, 64, 63), (77, 93, 131), (161, 160, 160)])
 def test_marches(shape):
     check(shape)
+
+
+# the x/y row kernel: several rows a workgroup (nx 5, 16, 24, 100, with the
+# last group cut by nz), one row, windows (nx 131, 257, 300, 515; one window
+# and several), y segments with a remainder, both dimensions
+@pytest.mark.parametrize("shape", [(9, 6, 5), (33, 40, 16), (17, 30, 24), (5, 50, 100), (6, 70, 131),
+                                   (3, 9, 256), (3, 7, 257), (8, 33, 300), (3, 3, 515), (1, 40, 64),
+                                   (1, 65, 130), (1, 33, 700)])
+@pytest.mark.parametrize("seg", [0, 7])
+def test_rows(shape, seg):
+    from pluto_amd import native
+    native.set_flux_kernel(1, seg)
+    try:
+        check(shape, dims=2 if shape[0] == 1 else 3)
+    finally:
+        native.set_flux_kernel()
