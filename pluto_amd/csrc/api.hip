@@ -780,6 +780,7 @@ static int enqueue_step_fused(pgpu_domain* d)
   const bool sig = d->sig_on;
   if (sig) rc = launch_sig_sweep(g, in1, d->sig, d->stream);
   if (!rc) rc = flux(1, in1, U, fd);
+  if (!rc && sig) rc = launch_vel_slopes(g, in1, d->sw, d->stream);
   if (!rc && sig) rc = launch_sig_emf(g, in1, d->sw, d->sig, d->stream);
   if (!rc) rc = launch_emf(g, in1, d->sw, d->e, d->stream, kt, fp32);
   // the FP32-flux path stores V1 (read only by stage 2's FP32 flux and EMF
@@ -791,6 +792,7 @@ static int enqueue_step_fused(pgpu_domain* d)
   if (rc) return rc;
   if (sig) rc = launch_sig_sweep(g, in2, d->sig, d->stream);
   if (!rc) rc = flux(2, in2, U, fd);
+  if (!rc && sig) rc = launch_vel_slopes(g, in2, d->sw, d->stream);
   if (!rc && sig) rc = launch_sig_emf(g, in2, d->sw, d->sig, d->stream);
   if (!rc) rc = launch_emf(g, in2, d->sw, d->e, d->stream, kt, fp32, fp32);
   if (!rc) rc = launch_ct_c2p(g, 2, d->e, fB, fA, oC, U, vn, V, d->flag, d->sc, d->stream, kt);

@@ -18,7 +18,7 @@
 //                     HLLD) from LDS, fluxes go to LDS, and each cell adds
 //                     -dt/dx (F_{i+1/2}-F_{i-1/2}) and the y counterpart to
 //                     its conservative state in registers.  Writes U, the
-//                     UCT_HLL face speeds and velocity slopes of its own
+//                     UCT_HLL face speeds of its own
 //                     faces/cells, and C_dt's x+y part.
 //   k_flux_z<STAGE>   one thread per (i,j) column marching up a z segment:
 //                     each cell's z PLM and each z interface is computed
@@ -50,8 +50,10 @@ __device__ __forceinline__ void face_store(double* a, long c, R v)
   else a[c] = v;
 }
 
-// what the flux kernels store per face for the EMF: the UCT_HLL data (face
-// speeds and velocity slopes), or the face EMFs from the normal fluxes of B
+// what the flux kernels store per face for the EMF: the UCT_HLL face speeds
+// (the EMF kernel reconstructs the velocity slopes; not storing them took
+// the x/y rows from 1255 to 1150 us and the z march from 653 to 600 at
+// 256^3), or the face EMFs from the normal fluxes of B
 // and the mass flux (ARITHMETIC, UCT0, UCT_CONTACT)
 constexpr int FACE_UCT_HLL = 0;
 constexpr int FACE_BFLUX = 1;
@@ -155,7 +157,7 @@ k_flux_xy(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScalars* sc
 
   // x interface between cells (ci-1, cj) and (ci, cj): cells ci-2 .. ci+1 at LDS x = tx .. tx+3
   {
-    R a[4][NV], vL[NV], vR[NV], vm0[NV], vpn[NV], vmn[NV], dvc[3];
+    R a[4][NV], vL[NV], vR[NV], vm0[NV], vpn[NV], vmn[NV];
     for (int s = 0; s < 4; s++)
 #pragma unroll
       for (int v = 0; v < NV; v++) a[s][v] = sv[v][ty + 2][tx + s];
@@ -163,8 +165,6 @@ k_flux_xy(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScalars* sc
     plm_cell(a[1], a[2], a[3], vpn, vmn);
 #pragma unroll
     for (int v = 0; v < NV; v++) vR[v] = vmn[v];
-#pragma unroll
-    for (int v = 0; v < 3; v++) dvc[v] = vL[VX1 + v] - vm0[VX1 + v];
     const int oi = wrap_any(ci - 1, g.nx), oj = wrap_any(cj, g.ny);   // owner cell of the face
     const long cf = plane + (long)oj * g.nx + oi;
     const R bface = R(in.b[0][cf]);
@@ -188,9 +188,6 @@ k_flux_xy(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScalars* sc
       } else {
         face_store(fd.SL[0], cf, max_ge(R(0), -r.SL));
         face_store(fd.SR[0], cf, max_ge(R(0), r.SR));
-        face_store(fd.dv[0][0], cf, dvc[0]);
-        face_store(fd.dv[0][1], cf, dvc[1]);
-        face_store(fd.dv[0][2], cf, dvc[2]);
       }
     }
     const double rm = double(r.mach);
@@ -198,7 +195,7 @@ k_flux_xy(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScalars* sc
   }
   // y interface between cells (ci, cj-1) and (ci, cj): rows cj-2 .. cj+1 at LDS y = ty .. ty+3
   {
-    R a[4][NV], vL[NV], vR[NV], vm0[NV], vpn[NV], vmn[NV], dvc[3];
+    R a[4][NV], vL[NV], vR[NV], vm0[NV], vpn[NV], vmn[NV];
     for (int s = 0; s < 4; s++)
 #pragma unroll
       for (int v = 0; v < NV; v++) a[s][v] = sv[v][ty + s][tx + 2];
@@ -206,8 +203,6 @@ k_flux_xy(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScalars* sc
     plm_cell(a[1], a[2], a[3], vpn, vmn);
 #pragma unroll
     for (int v = 0; v < NV; v++) vR[v] = vmn[v];
-#pragma unroll
-    for (int v = 0; v < 3; v++) dvc[v] = vL[VX1 + v] - vm0[VX1 + v];
     const int oi = wrap_any(ci, g.nx), oj = wrap_any(cj - 1, g.ny);   // owner cell of the face
     const long cf = plane + (long)oj * g.nx + oi;
     const R bface = R(in.b[1][cf]);
@@ -231,9 +226,6 @@ k_flux_xy(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScalars* sc
       } else {
         face_store(fd.SL[1], cf, max_ge(R(0), -r.SL));
         face_store(fd.SR[1], cf, max_ge(R(0), r.SR));
-        face_store(fd.dv[1][0], cf, dvc[0]);
-        face_store(fd.dv[1][1], cf, dvc[1]);
-        face_store(fd.dv[1][2], cf, dvc[2]);
       }
     }
     const double rm = double(r.mach);
@@ -333,7 +325,7 @@ k_flux_xy_items(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScala
   // box needs (tiles wider than the box) are skipped
   for (int item = tid; item < NXI + NYI; item += NT) {
     RiemannOut<R> r;
-    R vL[NV], vR[NV], dvc[3];
+    R vL[NV], vR[NV];
     R a[4][NV];
     int li, lj, own, gi, gj;
     if (item < NXI) {
@@ -353,8 +345,6 @@ k_flux_xy_items(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScala
       plm_cell(a[1], a[2], a[3], vpn, vmn);
 #pragma unroll
       for (int v = 0; v < NV; v++) vR[v] = vmn[v];
-#pragma unroll
-      for (int v = 0; v < 3; v++) dvc[v] = vL[VX1 + v] - vm0[VX1 + v];
       const long cf = plane + (long)wrap(gj, g.ny) * g.nx + wrap(gi, g.nx);
       const R bface = R(in.b[0][cf]);
       vL[BX1] = bface;
@@ -371,9 +361,6 @@ k_flux_xy_items(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScala
         const long c = plane + (long)gj * g.nx + gi;
         face_store(fd.SL[0], c, max_ge(R(0), -r.SL));
         face_store(fd.SR[0], c, max_ge(R(0), r.SR));
-        face_store(fd.dv[0][0], c, dvc[0]);
-        face_store(fd.dv[0][1], c, dvc[1]);
-        face_store(fd.dv[0][2], c, dvc[2]);
       }
     } else {
       const int it = item - NXI;
@@ -392,8 +379,6 @@ k_flux_xy_items(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScala
       plm_cell(a[1], a[2], a[3], vpn, vmn);
 #pragma unroll
       for (int v = 0; v < NV; v++) vR[v] = vmn[v];
-#pragma unroll
-      for (int v = 0; v < 3; v++) dvc[v] = vL[VX1 + v] - vm0[VX1 + v];
       const long cf = plane + (long)wrap(gj, g.ny) * g.nx + wrap(gi, g.nx);
       const R bface = R(in.b[1][cf]);
       vL[BX2] = bface;
@@ -410,9 +395,6 @@ k_flux_xy_items(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScala
         const long c = plane + (long)gj * g.nx + gi;
         face_store(fd.SL[1], c, max_ge(R(0), -r.SL));
         face_store(fd.SR[1], c, max_ge(R(0), r.SR));
-        face_store(fd.dv[1][0], c, dvc[0]);
-        face_store(fd.dv[1][1], c, dvc[1]);
-        face_store(fd.dv[1][2], c, dvc[2]);
       }
     }
     const double rm = double(r.mach);
@@ -620,16 +602,6 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
   // among them) before a barrier that publishes the copies
   auto wait_vm = [] { __builtin_amdgcn_s_waitcnt(0x0070); };   // vmcnt(0) lgkmcnt(0)
   auto rv = [&](int sl, int q, int ii) -> R { return R(ring[(sl * NV + q) * nt + ii]); };
-  // velocity slopes of the y reconstruction of cell (i, jj)
-  auto store_dvy = [&](int jj, const R* vp, const R* vm) {
-    if constexpr (E != FACE_BFLUX) {
-      const unsigned o = off8(jj);
-      fstore(fd.dv[1][0], o, vp[VX1] - vm[VX1]);
-      fstore(fd.dv[1][1], o, vp[VX2] - vm[VX2]);
-      fstore(fd.dv[1][2], o, vp[VX3] - vm[VX3]);
-    }
-  };
-
   stage_row(j0, 0);
   stage_row(j0 + 1, 1);
   // the y right-face state of cell (i, j0) and the y flux at j0-1/2
@@ -642,7 +614,6 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
     load(j0 + 1, w1);
     plm_cell(a, b, w0, vpb, vmb);      // cell (i, j0-1)
     plm_cell(b, w0, w1, vpy, vm0);     // cell (i, j0)
-    if (act) store_dvy(j0, vpy, vm0);
     R vL[NV], vR[NV];
 #pragma unroll
     for (int q = 0; q < NV; q++) {
@@ -709,13 +680,6 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
       // at the top of the row instead of sinking into a branch)
 #pragma unroll
       for (int q = 0; q < NV; q++) xp[q * nt + t] = q == BX1 ? bfx : vpx[q];
-      if (act) {
-        if constexpr (E != FACE_BFLUX) {
-          fstore(fd.dv[0][0], c, vpx[VX1] - vmx[VX1]);
-          fstore(fd.dv[0][1], c, vpx[VX2] - vmx[VX2]);
-          fstore(fd.dv[0][2], c, vpx[VX3] - vmx[VX3]);
-        }
-      }
     }
     __syncthreads();
     // row j+2 into the slot of row j-1 (last read before the barrier)
@@ -799,7 +763,6 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
       }
       plm_cell(a, b, w2, vpn, vmn);
     }
-    if (act && j + 1 < j1) store_dvy(j + 1, vpn, vmn);
     {
       R vL[NV], vR[NV];
 #pragma unroll
@@ -864,7 +827,7 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
 // length, so only the plane's last workgroup has idle lanes (rows cut into
 // 64-wide tiles left 31% of the lanes of a 133-cell row idle: 133^3 171 ->
 // 121 us a launch, 131 x 93 x 77 81 -> 53).  At 256^3 the march moves its
-// 195 B per cell at 5.0 TB/s, the rate of a large copy; small boxes are
+// 171 B per cell at 4.8 TB/s, the rate of a large copy; small boxes are
 // bound by the solves one after another along a segment (march_len).
 
 template <int STAGE, typename R, int S, int E, int V = 0>
@@ -899,9 +862,8 @@ k_flux_z(Geo g, StageIn in, Cons U, FaceData fd, const double* cdt_xy, int seg, 
       if constexpr (sizeof(R) == 4) at_byte(reinterpret_cast<float*>(a), o >> 1) = v;
       else at_byte(a, o) = v;
     };
-    // vb = v(k), vc = v(k+1); vp_k: right-face state of cell k, dv_k its
-    // velocity slopes
-    R vb[NV], vc[NV], vp_k[NV], dv_k[3];
+    // vb = v(k), vc = v(k+1); vp_k: right-face state of cell k
+    R vb[NV], vc[NV], vp_k[NV];
     R fprev[6], cmprev;
     {
       R va[NV], vm_k[NV], vp_n[NV], vm_n[NV];
@@ -932,8 +894,6 @@ k_flux_z(Geo g, StageIn in, Cons U, FaceData fd, const double* cdt_xy, int seg, 
       cmprev = r.cmax;
 #pragma unroll
       for (int q = 0; q < NV; q++) vp_k[q] = vp_n[q];   // cell k0
-#pragma unroll
-      for (int q = 0; q < 3; q++) dv_k[q] = vp_n[VX1 + q] - vm_n[VX1 + q];
     }
     // march: vb = v(k), vc = v(k+1)
     for (int k = k0; k < k1; k++) {
@@ -949,11 +909,6 @@ k_flux_z(Geo g, StageIn in, Cons U, FaceData fd, const double* cdt_xy, int seg, 
       for (int q = 0; q < 5; q++) u[q] = at_byte(U.u[q], c);
       if (STAGE == 1) cdt = at_byte(cdt_xy, c);
       plm_cell(vb, vc, vn, vp_n, vm_n);     // cell k+1
-      if constexpr (E != FACE_BFLUX) {
-        fstore(fd.dv[2][0], c, dv_k[0]);
-        fstore(fd.dv[2][1], c, dv_k[1]);
-        fstore(fd.dv[2][2], c, dv_k[2]);
-      }
       R vL[NV], vR[NV];
 #pragma unroll
       for (int q = 0; q < NV; q++) {
@@ -996,8 +951,6 @@ k_flux_z(Geo g, StageIn in, Cons U, FaceData fd, const double* cdt_xy, int seg, 
         vb[q] = vc[q];
         vc[q] = vn[q];
       }
-#pragma unroll
-      for (int q = 0; q < 3; q++) dv_k[q] = vp_n[VX1 + q] - vm_n[VX1 + q];
     }
   }
   block_max(mach, &sc->mach_max, red);

@@ -35,16 +35,17 @@ inline int march_len(int most, int line, W waves)
   return best;
 }
 
-// Per-face UCT_HLL speeds and per-cell velocity slopes written by the flux
-// kernels for the EMF kernel (same arrays as SweepOut's).
+// Per-face UCT_HLL speeds written by the flux kernels for the EMF kernel
+// (same arrays as SweepOut's; dv[direction][0]: the mass flux of the other
+// EMF averages).
 struct FaceData {
   double* SL[3];
   double* SR[3];
-  double* dv[3][3];   // dv[direction][velocity component]
+  double* dv[3][3];
 };
 
 // fp32_flux: PLM and HLLD in FP32 (states rounded from FP64 on load); the
-// flux differences and U are FP64; the face speeds and velocity slopes are
+// flux differences and U are FP64; the face speeds are
 // stored as float in the first half of fd's buffers (launch_emf with
 // f32_faces reads them).
 int launch_flux_fused(const Geo& g, int stage, bool fp32_flux, const StageIn& in, const Cons& U,

@@ -427,11 +427,12 @@ static bool enqueue_emf(const Geo& g, const StageIn& in, const Sweeps& sw, const
     PGPU_TIMED(KT_EMF, k_emf_faces<EMF_UCT0>, grid_of(g), kBlock, 0, s, g, in, sw, e);
   } else if (g.emf_avg == EMF_UCT_CONTACT) {
     PGPU_TIMED(KT_EMF, k_emf_faces<EMF_UCT_CONTACT>, grid_of(g), kBlock, 0, s, g, in, sw, e);
-  } else if ((g_emf_kernel || g.pz > 0) &&
+  } else if ((g_emf_kernel || g.pz > 0 || g.dims != 3) &&
              launch_emf_lds(g, in, sw, e, s, g_emf_kernel ? g_emf_kernel : 3, g_emf_lds_kz, kt,
                             f32_state ? 2 : (f32_faces ? 1 : 0))) {
     // LDS-staged z-march (the only EMF kernel for a stack of patches)
-  } else if (g.pz > 0) {
+  } else if (g.pz > 0 ||
+             launch_vel_slopes(g, in, sw, s, f32_state ? 2 : (f32_faces ? 1 : 0)) != 0) {
     return false;
   } else if (g.dims == 3 && (unsigned long long)g.n * 8ull < (1ull << 32)) {
     const dim3 b(g_emf_bx, g_emf_by, 1);

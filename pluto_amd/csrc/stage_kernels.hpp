@@ -192,12 +192,15 @@ int launch_c2p(const Geo& g, int stage, const Cons& U, const FaceIn& b, const St
 // values.
 int set_emf_tiling(int bx, int by, int kz);
 int set_emf_kernel(int kind, int kz);
-// LDS-staged UCT_HLL EMF (emf_lds.hip) for a 3D box with nx even, tile shape
-// 1 (64 x 4), 2 (32 x 4) or 3 (32 x 8), face data of type ft (0 double, 1
-// float, 2 float with an FP32 stage input); false when the box does not
-// qualify (the caller runs k_emf_z)
+// LDS-staged UCT_HLL EMF (emf_lds.hip), tile shape 1 (64 x 4), 2 (32 x 4) or
+// 3 (32 x 8), face data of type ft (0 double, 1 float, 2 float with an FP32
+// stage input); reconstructs the velocity slopes itself.  False when a field
+// is 4 GiB or more.
 bool launch_emf_lds(const Geo& g, const StageIn& in, const Sweeps& sw, const EdgeOut& e,
                     hipStream_t s, int shape, int kz, KernelTimer* kt, int ft = 0);
+// the PLM velocity slopes of the stage input into sw's dv arrays (which the
+// fused flux kernels do not write), for the kernels that read them there
+int launch_vel_slopes(const Geo& g, const StageIn& in, const Sweeps& sw, hipStream_t s, int ft = 0);
 
 // Branch signature of a stage (branch_sig.hip): hashes of the outcomes of
 // every piecewise operation, added into *acc.

@@ -74,3 +74,18 @@ def test_rows(shape, seg):
         check(shape, dims=2 if shape[0] == 1 else 3)
     finally:
         native.set_flux_kernel()
+
+
+# the LDS EMF: tiles cut at the row and plane ends, even rows (16-byte copies)
+# and odd ones (4-byte), boxes narrower than a tile, z segments with a
+# remainder, 2D
+@pytest.mark.parametrize("shape", [(3, 3, 3), (5, 9, 31), (17, 8, 32), (18, 7, 33), (6, 10, 34),
+                                   (33, 17, 66), (1, 3, 3), (1, 9, 32), (1, 25, 67)])
+@pytest.mark.parametrize("kind", [1, 2, 3])
+def test_emf_tiles(shape, kind):
+    from pluto_amd import native
+    native.set_emf_kernel(kind)
+    try:
+        check(shape, dims=2 if shape[0] == 1 else 3)
+    finally:
+        native.set_emf_kernel()
