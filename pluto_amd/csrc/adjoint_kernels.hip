@@ -840,8 +840,7 @@ static int adj_forward(pgpu_domain* d, const StepTape& T, double* const outB[3])
       fd2.dv[dd][c] = sw2.d[dd].dv[c];
     }
   }
-  int rc = launch_zero_flags(g, d->flag, s);
-  if (!rc) rc = launch_flux_fused(g, 1, false, in1, U, fd1, d->cdt, d->sc, s, nullptr);
+  int rc = launch_flux_fused(g, 1, false, in1, U, fd1, d->cdt, d->sc, s, nullptr);
   if (!rc) rc = launch_vel_slopes(g, in1, sw1, s);
   if (!rc) rc = launch_emf(g, in1, sw1, d->e, s, nullptr);
   if (!rc) rc = launch_ct_c2p(g, 1, d->e, fA, fA, oB, U, vn, V1, d->flag, d->sc, s, nullptr);

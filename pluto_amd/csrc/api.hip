@@ -778,6 +778,12 @@ static int enqueue_step_fused(pgpu_domain* d)
   int rc = enqueue_boundary(d, d->V, d->bA, 1);
   if (rc) return rc;
   const bool sig = d->sig_on;
+  StepEnds ends;   // the CT kernels clear the flags, move the NaN count and close the step
+  ends.on = 1;
+  ends.dims = g.dims;
+  ends.fixed_dt = d->fixed_dt;
+  ends.cfl = d->cfl;
+  ends.cfl_max_var = d->cfl_max_var;
   if (sig) rc = launch_sig_sweep(g, in1, d->sig, d->stream);
   if (!rc) rc = flux(1, in1, U, fd);
   if (!rc && sig) rc = launch_vel_slopes(g, in1, d->sw, d->stream);
@@ -785,7 +791,7 @@ static int enqueue_step_fused(pgpu_domain* d)
   if (!rc) rc = launch_emf(g, in1, d->sw, d->e, d->stream, kt, fp32);
   // the FP32-flux path stores V1 (read only by stage 2's FP32 flux and EMF
   // kernels) as float
-  if (!rc) rc = launch_ct_c2p(g, 1, d->e, fA, fA, oB, U, vn, V1, d->flag, d->sc, d->stream, kt, fp32);
+  if (!rc) rc = launch_ct_c2p(g, 1, d->e, fA, fA, oB, U, vn, V1, d->flag, d->sc, d->stream, kt, fp32, ends);
   // stage 2: V1, bB (+ V, bA for the blend) -> V, bC
   if (rc) return fail(PGPU_EDEVICE, "stage launch failed: %s", hipGetErrorString((hipError_t)rc));
   rc = enqueue_boundary(d, d->V1, d->bB, 2);
@@ -795,7 +801,7 @@ static int enqueue_step_fused(pgpu_domain* d)
   if (!rc && sig) rc = launch_vel_slopes(g, in2, d->sw, d->stream);
   if (!rc && sig) rc = launch_sig_emf(g, in2, d->sw, d->sig, d->stream);
   if (!rc) rc = launch_emf(g, in2, d->sw, d->e, d->stream, kt, fp32, fp32);
-  if (!rc) rc = launch_ct_c2p(g, 2, d->e, fB, fA, oC, U, vn, V, d->flag, d->sc, d->stream, kt);
+  if (!rc) rc = launch_ct_c2p(g, 2, d->e, fB, fA, oC, U, vn, V, d->flag, d->sc, d->stream, kt, false, ends);
   if (rc) return fail(PGPU_EDEVICE, "stage launch failed: %s", hipGetErrorString((hipError_t)rc));
   // the step's faces are in bC: rotate so that bA is the state again
   for (int a = 0; a < 3; a++) {
@@ -808,10 +814,10 @@ static int enqueue_step_fused(pgpu_domain* d)
 
 static int enqueue_step(pgpu_domain* d)
 {
+  if (d->pipeline != PGPU_PIPELINE_MODULAR && !d->tape_mode) return enqueue_step_fused(d);
   int rc = launch_zero_flags(d->g, d->flag, d->stream, d->sc);
   if (rc) return fail(PGPU_EDEVICE, "flag clear launch failed (%d)", rc);
-  rc = (d->pipeline == PGPU_PIPELINE_MODULAR || d->tape_mode) ? enqueue_step_modular(d)
-                                                              : enqueue_step_fused(d);
+  rc = enqueue_step_modular(d);
   if (rc) return rc;
   KernelTimer* kt = d->timer;
   if (kt) kt->begin(KT_STEP_END, d->stream);

@@ -40,17 +40,41 @@ __device__ __forceinline__ double new_face(const Geo& g, const EdgeOut& e, const
   return b;
 }
 
+// dt of the step, and the step's ends in the CT kernels.  Stage 1 of a step
+// takes the previous step's output NaN count and leaves dt in dt_step for
+// stage 2, where the first thread closes the step at once: no other thread
+// of that launch reads what it writes, and every reduction it closes was
+// finished by the flux kernels.  Two launches per step less (32^3 as three
+// boxes in turn 684 -> 580 us for 16 steps; counting the workgroups that have read dt instead
+// took back all of it on a 512^2 plane, 1024 additions to one address).
+template <int STAGE>
+__device__ __forceinline__ double step_dt(const StepEnds& ends, DevScalars* sc, unsigned tid)
+{
+  const double dt = STAGE == 2 && ends.on ? sc->dt_step : sc->dt;
+  if (ends.on && tid == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
+    if (STAGE == 1) {
+      sc->dt_step = dt;
+      const unsigned n = sc->nan_next;
+      sc->nan_next = 0;
+      if (n) atomicAdd(&sc->nan_cells, n);
+    } else {
+      close_step(sc, ends.dims, ends.cfl, ends.cfl_max_var, ends.fixed_dt);
+    }
+  }
+  return dt;
+}
+
 template <int STAGE, bool F32OUT>
 __global__ void __launch_bounds__(256) k_ct_c2p(Geo g, EdgeOut e, FaceIn bin, FaceIn b0,
                                                 FaceOut bout, Cons U, StageIn vn, Prims Vout,
-                                                unsigned char* flag, DevScalars* sc)
+                                                unsigned char* flag, DevScalars* sc, StepEnds ends)
 {
+  const double dt = step_dt<STAGE>(ends, sc, threadIdx.x + blockDim.x * threadIdx.y);
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int j = blockIdx.y * blockDim.y + threadIdx.y;
   const int k = blockIdx.z;
   if (i >= g.nx || j >= g.ny) return;
   const long c = ((long)k * g.ny + j) * g.nx + i;
-  const double dt = sc->dt;
   const double dtx = dt / g.dx[0], dty = dt / g.dx[1], dtz = dt / g.dx[2];
   const int im = (i == 0 ? g.nx - 1 : i - 1), jm = (j == 0 ? g.ny - 1 : j - 1);
   const int km = (k == 0 ? g.nz - 1 : k - 1);
@@ -98,9 +122,10 @@ __global__ void __launch_bounds__(256) k_ct_c2p(Geo g, EdgeOut e, FaceIn bin, Fa
       U.u[0][c] = u[RHO];
       U.u[4][c] = u[ENG];
     }
-    flag[c] |= f;
+    if (STAGE == 2) flag[c] |= f;
     if (in_dom(g, i, j, k)) atomicAdd(&sc->fail_cells, 1u);
   }
+  if (STAGE == 1) flag[c] = f;   // (a step's flags start here)
   if (has_nan(v) && in_dom(g, i, j, k)) atomicAdd(STAGE == 1 ? &sc->nan_cells : &sc->nan_next, 1u);
 }
 
@@ -127,14 +152,15 @@ __device__ __forceinline__ double ct_face(double bin, double b0, double r)
 template <int STAGE, bool F32OUT>
 __global__ void __launch_bounds__(256) k_ct_c2p_z(Geo g, EdgeOut e, FaceIn bin, FaceIn b0,
                                                   FaceOut bout, Cons U, StageIn vn, Prims Vout,
-                                                  unsigned char* flag, DevScalars* sc, int kz)
+                                                  unsigned char* flag, DevScalars* sc, int kz,
+                                                  StepEnds ends)
 {
   const unsigned col = blockIdx.x * blockDim.x + threadIdx.x;   // cell of the plane
-  if (col >= (unsigned)g.nx * (unsigned)g.ny) return;
-  const int j = (int)(col / (unsigned)g.nx), i = (int)(col - (unsigned)j * (unsigned)g.nx);
   const ZSeg zs = zseg(g, blockIdx.y, kz);   // (a patch of a stack: z periodic within it)
   sc = scal(sc, g, zs.k0);
-  const double dt = sc->dt;
+  const double dt = step_dt<STAGE>(ends, sc, threadIdx.x);
+  if (col >= (unsigned)g.nx * (unsigned)g.ny) return;
+  const int j = (int)(col / (unsigned)g.nx), i = (int)(col - (unsigned)j * (unsigned)g.nx);
   const double dtx = dt / g.dx[0], dty = dt / g.dx[1], dtz = dt / g.dx[2];
   const unsigned rowb = (unsigned)g.nx * 8u;
   const unsigned planeb = rowb * (unsigned)g.ny;
@@ -208,9 +234,10 @@ __global__ void __launch_bounds__(256) k_ct_c2p_z(Geo g, EdgeOut e, FaceIn bin, 
         at_byte(U.u[0], c) = u[RHO];
         at_byte(U.u[4], c) = u[ENG];
       }
-      flag[(unsigned long)(c >> 3)] |= f;
+      if (STAGE == 2) flag[(unsigned long)(c >> 3)] |= f;
       if (in_dom(g, i, j, k)) atomicAdd(&sc->fail_cells, 1u);
     }
+    if (STAGE == 1) flag[(unsigned long)(c >> 3)] = f;   // (a step's flags start here)
     if (has_nan(v) && in_dom(g, i, j, k))
       atomicAdd(STAGE == 1 ? &sc->nan_cells : &sc->nan_next, 1u);
     ey_p = ey;
@@ -224,7 +251,7 @@ __global__ void __launch_bounds__(256) k_ct_c2p_z(Geo g, EdgeOut e, FaceIn bin, 
 int launch_ct_c2p(const Geo& g, int stage, const EdgeOut& e, const FaceIn& bin, const FaceIn& b0,
                   const FaceOut& bout, const Cons& U, const StageIn& vn, const Prims& Vout,
                   unsigned char* flag, DevScalars* sc, hipStream_t s, KernelTimer* kt,
-                  bool f32_out)
+                  bool f32_out, const StepEnds& ends)
 {
   if (f32_out && stage != 1) return (int)hipErrorInvalidValue;
   const bool zmarch = g.dims == 3 && (unsigned long long)g.n * 8ull < (1ull << 32);
@@ -243,17 +270,17 @@ int launch_ct_c2p(const Geo& g, int stage, const EdgeOut& e, const FaceIn& bin, 
     while (kz > 1 && (long)wgs * zblocks(g, kz) < 2048) kz /= 2;
     const dim3 gz(wgs, zblocks(g, kz)), bz(256);
     if (f32_out)
-      hipLaunchKernelGGL((k_ct_c2p_z<1, true>), gz, bz, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, kz);
+      hipLaunchKernelGGL((k_ct_c2p_z<1, true>), gz, bz, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, kz, ends);
     else if (stage == 1)
-      hipLaunchKernelGGL((k_ct_c2p_z<1, false>), gz, bz, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, kz);
+      hipLaunchKernelGGL((k_ct_c2p_z<1, false>), gz, bz, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, kz, ends);
     else
-      hipLaunchKernelGGL((k_ct_c2p_z<2, false>), gz, bz, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, kz);
+      hipLaunchKernelGGL((k_ct_c2p_z<2, false>), gz, bz, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, kz, ends);
   } else if (f32_out) {
-    hipLaunchKernelGGL((k_ct_c2p<1, true>), gr, b, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc);
+    hipLaunchKernelGGL((k_ct_c2p<1, true>), gr, b, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, ends);
   } else if (stage == 1) {
-    hipLaunchKernelGGL((k_ct_c2p<1, false>), gr, b, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc);
+    hipLaunchKernelGGL((k_ct_c2p<1, false>), gr, b, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, ends);
   } else {
-    hipLaunchKernelGGL((k_ct_c2p<2, false>), gr, b, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc);
+    hipLaunchKernelGGL((k_ct_c2p<2, false>), gr, b, 0, s, g, e, bin, b0, bout, U, vn, Vout, flag, sc, ends);
   }
   if (kt) kt->end(KT_CT, s);
   return (int)hipGetLastError();

@@ -493,6 +493,50 @@ __device__ __forceinline__ void emf_faces_cell(const Geo& g, const Cell& p, cons
 }
 
 // ---------------------------------------------------------------------
+// step end
+// ---------------------------------------------------------------------
+
+// One thread: close the step.  invDt_hyp = max(C_dt)/DIMENSIONS
+// (update_stage.c:310-311); dt_next per NextTimeStep (main.c:462-532).
+__device__ __forceinline__ void close_step(DevScalars* sc, int dims, double cfl, double cfl_max_var,
+                                           int fixed_dt)
+{
+  double inv = __longlong_as_double((long long)sc->invdt_max);
+  inv /= (double)dims;
+  const double mach = __longlong_as_double((long long)sc->mach_max);
+  const double dt = sc->dt;
+  sc->cdt_raw_last = __longlong_as_double((long long)sc->invdt_max);
+  sc->invdt_last = inv;
+  sc->mach_last = mach;
+  sc->dt_last = dt;
+  sc->time += dt;
+  sc->step += 1;
+  if (!fixed_dt) {
+    double dt_hyp = 1.0 / inv;
+    dt_hyp *= cfl;
+    double dtnext = dt_hyp;
+    const double cap = cfl_max_var * dt;
+    dtnext = dtnext <= cap ? dtnext : cap;
+    // dt too small (main.c:534-543): PLUTO quits there; record the first
+    // such dt and take no more time in the steps already enqueued
+    if (dtnext < sc->first_dt * 1.e-9) {
+      if (!sc->dt_small) sc->dt_small_value = dtnext;
+      sc->dt_small = 1;
+      dtnext = 0.0;
+    }
+    sc->dt = dtnext;
+  }
+  const long long h = sc->step - 1;
+  if (h >= 0 && h < DT_HISTORY) {
+    sc->dt_hist[h] = dt;
+    sc->invdt_hist[h] = inv;
+    sc->mach_hist[h] = mach;
+  }
+  sc->invdt_max = 0ull;
+  sc->mach_max = 0ull;
+}
+
+// ---------------------------------------------------------------------
 // ct, c2p
 // ---------------------------------------------------------------------
 

@@ -116,11 +116,21 @@ struct DevScalars {
   unsigned int nan_next;            // NaN cells of the last stage-2 output, the next
                                     // step's input: added to nan_cells when it starts
   unsigned int dt_small;            // NextTimeStep's stop (main.c:534-543) was reached
+  double dt_step;                   // dt of the step as its stage 1 left it for stage 2's CT
   double first_dt;                  // the run's first dt (ini->first_dt)
   double dt_small_value;            // the dt that was too small
   double dt_hist[DT_HISTORY];
   double invdt_hist[DT_HISTORY];
   double mach_hist[DT_HISTORY];
+};
+
+// What the CT kernels of a fused step do at its ends besides their work:
+// stage 1 takes the previous step's output NaN count into the stage-input
+// count (start), stage 2 closes the step (end: NextTimeStep's rule).
+struct StepEnds {
+  int on = 0;
+  int dims = 3, fixed_dt = 0;
+  double cfl = 0.0, cfl_max_var = 0.0;
 };
 
 struct StageIn {
