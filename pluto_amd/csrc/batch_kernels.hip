@@ -377,13 +377,6 @@ __global__ void k_batch_post(int nf, const int* ids, PatchScalars* ps, const cha
   }
 }
 
-// flags of the stacked zones cleared (a kernel: no memset node in the graph)
-__global__ void k_batch_clear_flags(unsigned char* flag, long n)
-{
-  for (long c = (long)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (long)gridDim.x * blockDim.x)
-    flag[c] = 0;
-}
-
 // the step's faces, written to a third set by the fused stage 2 (its output
 // may not alias its inputs), back into the state's faces
 __global__ void k_batch_copy_faces(const double* c0, const double* c1, const double* c2, double* a0,
@@ -422,8 +415,6 @@ struct pgpu_batch {
   int threads = 256;     // workgroup size
   int groups = 0;        // resident workgroups
   int tile[3] = {0, 0, 0};   // cell tile of a pass (0: linear)
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
   double cfl = 0.4, cfl_max_var = 1.1;
   int fixed_dt = 0;
   // stacked mode: the patches with stack_edge() edges come first in every
@@ -442,80 +433,133 @@ struct pgpu_batch {
   char* d_heads = nullptr;       // [nfused] scalars (DevScalars before the histories)
   long head_bytes = 0;
   int stacked_now = 0;           // the captured step runs the stacks
+  // A step of the batch as independent branches, each a linear graph on a
+  // stream of its own (branch 0: the batch's): the stacks dealt out by their
+  // zones, and the persistent kernel's patches.  No branch reads what another
+  // writes, so they meet only at the ends of a run.
+  struct Branch {
+    hipStream_t s = nullptr;
+    hipEvent_t ev = nullptr;
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+  };
+  std::vector<Branch> br;
+  int nbr = 0;                   // branches of the captured step
 };
 
-// one stage of every stack through the fused kernels
-static int enqueue_stacks(pgpu_batch* b, int stage)
+// one stage of a stack through the fused kernels
+static int enqueue_stack(pgpu_batch* b, const pgpu_batch::Stack& st, int stage, hipStream_t s)
 {
   const BatchArrays& A = b->A;
-  for (const auto& st : b->stacks) {
-    const long o = st.off;
-    Geo g;
-    g.nx = g.ny = st.n;
-    g.nz = st.count * st.n;
-    g.dims = 3;
-    g.n = (long)st.count * st.n * st.n * st.n;
-    for (int a = 0; a < 3; a++) {
-      g.dx[a] = 1.0 / st.n;
-      g.inv_dx[a] = 1.0 / g.dx[a];
-    }
-    g.gamma = b->gamma;
-    g.gmm1 = b->gamma - 1.0;
-    g.pz = st.n;
-    g.sc_stride = b->head_bytes;
-    DevScalars* sc = reinterpret_cast<DevScalars*>(b->d_heads + (long)st.first * b->head_bytes);
-    StageIn in, vn;
-    for (int q = 0; q < 8; q++) {
-      in.V[q] = (stage == 1 ? A.V[q] : A.V1[q]) + o;
-      vn.V[q] = A.V[q] + o;
-    }
-    for (int a = 0; a < 3; a++) {
-      in.b[a] = (stage == 1 ? A.bA[a] : A.bB[a]) + o;
-      vn.b[a] = A.bA[a] + o;
-    }
-    Cons U;
-    for (int q = 0; q < 5; q++) U.u[q] = A.U[q] + o;
-    Sweeps sw;
-    FaceData fd;
-    for (int a = 0; a < 3; a++) {
-      for (int q = 0; q < 5; q++) sw.d[a].F[q] = A.sw[a][q] + o;
-      sw.d[a].P = A.sw[a][5] + o;
-      sw.d[a].SL = fd.SL[a] = A.sw[a][6] + o;
-      sw.d[a].SR = fd.SR[a] = A.sw[a][7] + o;
-      sw.d[a].cm = A.sw[a][8] + o;
-      for (int k = 0; k < 3; k++) sw.d[a].dv[k] = fd.dv[a][k] = A.sw[a][9 + k] + o;
-    }
-    double* cdt = A.sw[0][0] + o;   // (the flux arrays of the modular sweeps are free here)
-    EdgeOut e;
-    e.ex = A.e[0] + o;
-    e.ey = A.e[1] + o;
-    e.ez = A.e[2] + o;
-    FaceIn fA, fB;
-    FaceOut oB, oC;
-    for (int a = 0; a < 3; a++) {
-      fA.b[a] = A.bA[a] + o;
-      fB.b[a] = A.bB[a] + o;
-      oB.b[a] = A.bB[a] + o;
-      oC.b[a] = A.sw[1][a] + o;   // third face set, copied back into bA after the step
-    }
-    Prims Vout;
-    for (int q = 0; q < 8; q++) Vout.v[q] = (stage == 1 ? A.V1[q] : A.V[q]) + o;
-    int rc = launch_flux_fused(g, stage, false, in, U, fd, cdt, sc, b->stream, nullptr);
-    if (!rc) rc = launch_emf(g, in, sw, e, b->stream, nullptr);
-    if (!rc)
-      rc = stage == 1 ? launch_ct_c2p(g, 1, e, fA, fA, oB, U, vn, Vout, A.flag + o, sc, b->stream, nullptr)
-                      : launch_ct_c2p(g, 2, e, fB, fA, oC, U, vn, Vout, A.flag + o, sc, b->stream, nullptr);
-    if (rc) return rc;
+  const long o = st.off;
+  Geo g;
+  g.nx = g.ny = st.n;
+  g.nz = st.count * st.n;
+  g.dims = 3;
+  g.n = (long)st.count * st.n * st.n * st.n;
+  for (int a = 0; a < 3; a++) {
+    g.dx[a] = 1.0 / st.n;
+    g.inv_dx[a] = 1.0 / g.dx[a];
   }
+  g.gamma = b->gamma;
+  g.gmm1 = b->gamma - 1.0;
+  g.pz = st.n;
+  g.sc_stride = b->head_bytes;
+  DevScalars* sc = reinterpret_cast<DevScalars*>(b->d_heads + (long)st.first * b->head_bytes);
+  StageIn in, vn;
+  for (int q = 0; q < 8; q++) {
+    in.V[q] = (stage == 1 ? A.V[q] : A.V1[q]) + o;
+    vn.V[q] = A.V[q] + o;
+  }
+  for (int a = 0; a < 3; a++) {
+    in.b[a] = (stage == 1 ? A.bA[a] : A.bB[a]) + o;
+    vn.b[a] = A.bA[a] + o;
+  }
+  Cons U;
+  for (int q = 0; q < 5; q++) U.u[q] = A.U[q] + o;
+  Sweeps sw;
+  FaceData fd;
+  for (int a = 0; a < 3; a++) {
+    for (int q = 0; q < 5; q++) sw.d[a].F[q] = A.sw[a][q] + o;
+    sw.d[a].P = A.sw[a][5] + o;
+    sw.d[a].SL = fd.SL[a] = A.sw[a][6] + o;
+    sw.d[a].SR = fd.SR[a] = A.sw[a][7] + o;
+    sw.d[a].cm = A.sw[a][8] + o;
+    for (int k = 0; k < 3; k++) sw.d[a].dv[k] = fd.dv[a][k] = A.sw[a][9 + k] + o;
+  }
+  double* cdt = A.sw[0][0] + o;   // (the flux arrays of the modular sweeps are free here)
+  EdgeOut e;
+  e.ex = A.e[0] + o;
+  e.ey = A.e[1] + o;
+  e.ez = A.e[2] + o;
+  FaceIn fA, fB;
+  FaceOut oB, oC;
+  for (int a = 0; a < 3; a++) {
+    fA.b[a] = A.bA[a] + o;
+    fB.b[a] = A.bB[a] + o;
+    oB.b[a] = A.bB[a] + o;
+    oC.b[a] = A.sw[1][a] + o;   // third face set, copied back into bA after the step
+  }
+  Prims Vout;
+  for (int q = 0; q < 8; q++) Vout.v[q] = (stage == 1 ? A.V1[q] : A.V[q]) + o;
+  int rc = launch_flux_fused(g, stage, false, in, U, fd, cdt, sc, s, nullptr);
+  if (!rc) rc = launch_emf(g, in, sw, e, s, nullptr);
+  if (!rc)
+    rc = stage == 1 ? launch_ct_c2p(g, 1, e, fA, fA, oB, U, vn, Vout, A.flag + o, sc, s, nullptr)
+                    : launch_ct_c2p(g, 2, e, fB, fA, oC, U, vn, Vout, A.flag + o, sc, s, nullptr);
+  if (rc) return rc;
   return 0;
+}
+
+static void drop_graphs(pgpu_batch* b)
+{
+  for (auto& r : b->br) {
+    if (r.exec) (void)hipGraphExecDestroy(r.exec);
+    if (r.graph) (void)hipGraphDestroy(r.graph);
+    r.exec = nullptr;
+    r.graph = nullptr;
+  }
+  b->nbr = 0;
+}
+
+// A whole step of stack st on stream s.
+static int enqueue_stack_step(pgpu_batch* b, const pgpu_batch::Stack& st, hipStream_t s)
+{
+  const int nfb = (st.count + 255) / 256;
+  const int* ids = b->d_fused_ids + st.first;
+  char* heads = b->d_heads + (long)st.first * b->head_bytes;
+  const long o = st.off, z = (long)st.count * st.n * st.n * st.n;
+  double* const* c = b->A.sw[1];
+  hipLaunchKernelGGL(k_batch_pre, dim3(nfb), dim3(256), 0, s, st.count, ids, b->d_ps, heads, b->head_bytes);
+  int rc = enqueue_stack(b, st, 1, s);
+  if (!rc) rc = enqueue_stack(b, st, 2, s);
+  if (rc) return rc;
+  const long nw = (z + 255) / 256;
+  hipLaunchKernelGGL(k_batch_copy_faces, dim3((unsigned)(nw < 4096 ? nw : 4096)), dim3(256), 0, s, c[0] + o,
+                     c[1] + o, c[2] + o, b->A.bA[0] + o, b->A.bA[1] + o, b->A.bA[2] + o, z);
+  hipLaunchKernelGGL(k_batch_post, dim3(nfb), dim3(256), 0, s, st.count, ids, b->d_ps, heads, b->head_bytes,
+                     b->cfl, b->cfl_max_var, b->fixed_dt);
+  return (int)hipGetLastError();
+}
+
+static void enqueue_persistent(pgpu_batch* b, const BatchCtl& C, hipStream_t s)
+{
+  if (C.npatch <= 0) return;
+  const dim3 g(b->groups), t(b->threads);
+  if (b->threads <= 512) {
+    hipLaunchKernelGGL((k_batch_stage<1, 512>), g, t, 0, s, b->A, C);
+    hipLaunchKernelGGL((k_batch_stage<2, 512>), g, t, 0, s, b->A, C);
+  } else {
+    hipLaunchKernelGGL((k_batch_stage<1, 1024>), g, t, 0, s, b->A, C);
+    hipLaunchKernelGGL((k_batch_stage<2, 1024>), g, t, 0, s, b->A, C);
+  }
 }
 
 static int batch_capture(pgpu_batch* b)
 {
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
-  if (b->graph) (void)hipGraphDestroy(b->graph);
-  b->exec = nullptr;
-  b->graph = nullptr;
+  // (no graph goes while a replay of it is under way)
+  if (hipStreamSynchronize(b->stream) != hipSuccess) return fail(PGPU_EDEVICE, "stream synchronisation failed");
+  drop_graphs(b);
   b->C.cfl = b->cfl;
   b->C.cfl_max_var = b->cfl_max_var;
   b->C.fixed_dt = b->fixed_dt;
@@ -531,40 +575,40 @@ static int batch_capture(pgpu_batch* b)
     C.order = b->d_rest_order;
     C.npatch = b->nrest;
   }
-  hipError_t err = hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal);
-  if (err != hipSuccess) return fail(PGPU_EDEVICE, "hipStreamBeginCapture: %s", hipGetErrorString(err));
-  int rc = 0;
-  auto persistent = [&](int stage) {
-    if (C.npatch <= 0) return;
-    if (b->threads <= 512) {
-      if (stage == 1) hipLaunchKernelGGL((k_batch_stage<1, 512>), dim3(b->groups), dim3(b->threads), 0, b->stream, b->A, C);
-      else hipLaunchKernelGGL((k_batch_stage<2, 512>), dim3(b->groups), dim3(b->threads), 0, b->stream, b->A, C);
-    } else {
-      if (stage == 1) hipLaunchKernelGGL((k_batch_stage<1, 1024>), dim3(b->groups), dim3(b->threads), 0, b->stream, b->A, C);
-      else hipLaunchKernelGGL((k_batch_stage<2, 1024>), dim3(b->groups), dim3(b->threads), 0, b->stream, b->A, C);
-    }
-  };
-  const int nfb = (b->nfused + 255) / 256;
+  // the stacks, the largest first, each to the branch with the fewest zones;
+  // the persistent kernel, slower per zone, on the last branch
+  const int nbr = stacked ? (int)b->br.size() : 1;
+  std::vector<std::vector<int>> deal(nbr);
   if (stacked) {
-    hipLaunchKernelGGL(k_batch_pre, dim3(nfb), dim3(256), 0, b->stream, b->nfused, b->d_fused_ids,
-                       b->d_ps, b->d_heads, b->head_bytes);
-    hipLaunchKernelGGL(k_batch_clear_flags, dim3(2048), dim3(256), 0, b->stream, b->A.flag, b->zfused);
+    std::vector<long> load(nbr, 0);
+    auto zones = [&](int q) {
+      const auto& st = b->stacks[q];
+      return (long)st.count * st.n * st.n * st.n;
+    };
+    if (b->nrest) load[nbr - 1] = 2 * (b->zones - b->zfused);
+    std::vector<int> ord(b->stacks.size());
+    std::iota(ord.begin(), ord.end(), 0);
+    std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return zones(x) > zones(y); });
+    for (int q : ord) {
+      const int r = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+      deal[r].push_back(q);
+      load[r] += zones(q);
+    }
   }
-  persistent(1);
-  if (stacked) rc = enqueue_stacks(b, 1);
-  persistent(2);
-  if (stacked && !rc) rc = enqueue_stacks(b, 2);
-  if (stacked && !rc) {
-    hipLaunchKernelGGL(k_batch_copy_faces, dim3(4096), dim3(256), 0, b->stream, b->A.sw[1][0], b->A.sw[1][1],
-                       b->A.sw[1][2], b->A.bA[0], b->A.bA[1], b->A.bA[2], b->zfused);
-    hipLaunchKernelGGL(k_batch_post, dim3(nfb), dim3(256), 0, b->stream, b->nfused, b->d_fused_ids,
-                       b->d_ps, b->d_heads, b->head_bytes, b->cfl, b->cfl_max_var, b->fixed_dt);
+  for (int r = 0; r < nbr; r++) {
+    auto& B = b->br[r];
+    hipError_t err = hipStreamBeginCapture(B.s, hipStreamCaptureModeThreadLocal);
+    if (err != hipSuccess) return fail(PGPU_EDEVICE, "hipStreamBeginCapture: %s", hipGetErrorString(err));
+    int rc = 0;
+    if (r == nbr - 1) enqueue_persistent(b, C, B.s);
+    for (size_t q = 0; q < deal[r].size() && !rc; q++) rc = enqueue_stack_step(b, b->stacks[deal[r][q]], B.s);
+    err = hipStreamEndCapture(B.s, &B.graph);
+    if (rc) return fail(PGPU_EDEVICE, "stacked stage launch failed (%d)", rc);
+    if (err != hipSuccess) return fail(PGPU_EDEVICE, "hipStreamEndCapture: %s", hipGetErrorString(err));
+    err = hipGraphInstantiate(&B.exec, B.graph, nullptr, nullptr, 0);
+    if (err != hipSuccess) return fail(PGPU_EDEVICE, "hipGraphInstantiate: %s", hipGetErrorString(err));
   }
-  err = hipStreamEndCapture(b->stream, &b->graph);
-  if (rc) return fail(PGPU_EDEVICE, "stacked stage launch failed (%d)", rc);
-  if (err != hipSuccess) return fail(PGPU_EDEVICE, "hipStreamEndCapture: %s", hipGetErrorString(err));
-  err = hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0);
-  if (err != hipSuccess) return fail(PGPU_EDEVICE, "hipGraphInstantiate: %s", hipGetErrorString(err));
+  b->nbr = nbr;
   return PGPU_OK;
 }
 
@@ -698,6 +742,19 @@ extern "C" int pgpu_batch_create(int npatch, const int* edge, double gamma, pgpu
     pgpu_batch_destroy(b);
     return fail(PGPU_EDEVICE, "batch set-up failed: %s", hipGetErrorString(err));
   }
+  // one branch per stack and one for the other patches, at most four (the
+  // hardware queues of a process)
+  const size_t want = b->stacks.size() + (b->nrest ? 1 : 0);
+  b->br.resize(want < 1 ? 1 : (want > 4 ? 4 : want));
+  for (size_t q = 0; q < b->br.size() && err == hipSuccess; q++) {
+    if (q == 0) b->br[q].s = b->stream;
+    else err = hipStreamCreateWithFlags(&b->br[q].s, hipStreamNonBlocking);
+    if (err == hipSuccess) err = hipEventCreateWithFlags(&b->br[q].ev, hipEventDisableTiming);
+  }
+  if (err != hipSuccess) {
+    pgpu_batch_destroy(b);
+    return fail(PGPU_EDEVICE, "batch streams: %s", hipGetErrorString(err));
+  }
   b->C.pd = b->d_pd;
   b->C.order = b->d_order;
   b->C.ps = b->d_ps;
@@ -719,8 +776,7 @@ extern "C" int pgpu_batch_destroy(pgpu_batch* b)
 {
   if (!b) return PGPU_OK;
   if (b->stream) (void)hipStreamSynchronize(b->stream);
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
-  if (b->graph) (void)hipGraphDestroy(b->graph);
+  drop_graphs(b);
   if (b->block) (void)hipFree(b->block);
   if (b->d_pd) (void)hipFree(b->d_pd);
   if (b->d_order) (void)hipFree(b->d_order);
@@ -729,6 +785,10 @@ extern "C" int pgpu_batch_destroy(pgpu_batch* b)
   if (b->d_fused_ids) (void)hipFree(b->d_fused_ids);
   if (b->d_rest_order) (void)hipFree(b->d_rest_order);
   if (b->d_heads) (void)hipFree(b->d_heads);
+  for (size_t q = 0; q < b->br.size(); q++) {
+    if (b->br[q].ev) (void)hipEventDestroy(b->br[q].ev);
+    if (q > 0 && b->br[q].s) (void)hipStreamDestroy(b->br[q].s);
+  }
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
   return PGPU_OK;
@@ -811,10 +871,24 @@ extern "C" int pgpu_batch_set_dt(pgpu_batch* b, double dt, double cfl, double cf
 extern "C" int pgpu_batch_run(pgpu_batch* b, int nsteps)
 {
   if (!b) return fail(PGPU_EINVAL, "batch is NULL");
-  for (int s = 0; s < nsteps; s++) {
-    const hipError_t err = hipGraphLaunch(b->exec, b->stream);
-    if (err != hipSuccess) return fail(PGPU_EDEVICE, "hipGraphLaunch: %s", hipGetErrorString(err));
+  if (b->nbr < 1) return fail(PGPU_EINVAL, "the batch has no captured step");
+  if (nsteps < 1) return PGPU_OK;
+  // the branches start after what the batch's stream holds and end in it
+  hipError_t err = hipSuccess;
+  if (b->nbr > 1) {
+    err = hipEventRecord(b->br[0].ev, b->stream);
+    for (int r = 1; r < b->nbr && err == hipSuccess; r++) err = hipStreamWaitEvent(b->br[r].s, b->br[0].ev, 0);
   }
+  for (int s = 0; s < nsteps && err == hipSuccess; s++)
+    for (int r = 0; r < b->nbr && err == hipSuccess; r++) err = hipGraphLaunch(b->br[r].exec, b->br[r].s);
+  hipError_t join = hipSuccess;
+  for (int r = 1; r < b->nbr; r++) {
+    hipError_t e = hipEventRecord(b->br[r].ev, b->br[r].s);
+    if (e == hipSuccess) e = hipStreamWaitEvent(b->stream, b->br[r].ev, 0);
+    if (e != hipSuccess) join = e;
+  }
+  if (err == hipSuccess) err = join;
+  if (err != hipSuccess) return fail(PGPU_EDEVICE, "hipGraphLaunch: %s", hipGetErrorString(err));
   return PGPU_OK;
 }
 

@@ -201,3 +201,30 @@ def test_stacked_mode_switches(native):
     with pytest.raises(native.PGPUError):
         b.set_mode(2)
     b.close()
+
+
+@pytest.mark.parametrize("edges", [[16] * 3, [8, 16, 12, 20, 24, 6, 8, 16], [16, 9, 12, 20, 7, 8, 10, 11]])
+def test_batch_branches(native, edges):
+    """Stacks on one branch and on four, with patches of the persistent
+    kernel beside them: several runs with reads between them equal the
+    persistent mode's single run."""
+    _say("case: batch branches %s" % edges)
+    states = [P.random_mhd_3d(n, seed=700 + p) for p, n in enumerate(edges)]
+    a, b = native.Batch(edges), native.Batch(edges)
+    b.set_mode(0)
+    for p, st in enumerate(states):
+        a.set_patch(p, st)
+        b.set_patch(p, st)
+    a.set_dt(1e-3)
+    b.set_dt(1e-3)
+    for n in (1, 3, 0, 2):
+        a.run(n)
+        a.get_patch(len(edges) - 1)
+    b.run(6)
+    a.sync()
+    b.sync()
+    for p in range(len(edges)):
+        assert_states_equal(a.get_patch(p), b.get_patch(p), "patch %d of %s" % (p, edges))
+        assert a.scalars(p) == b.scalars(p)
+    a.close()
+    b.close()
