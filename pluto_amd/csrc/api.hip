@@ -635,6 +635,11 @@ static int enqueue_boundary(pgpu_domain* d, double* const* v, double* const* b, 
   if (kt) kt->begin(KT_BOUNDARY, d->stream);
   int rc = 0;
   for (int is = 0; is < 6 && !rc; is++) {
+    if ((is & 1) == 0 && d->bound[is] != BOUND_USERDEF && d->bound[is + 1] != BOUND_USERDEF) {
+      rc = launch_boundary_axis(d->gb, is / 2, &d->bound[is], v, b, nullptr, d->area, d->stream);
+      is++;
+      continue;
+    }
     if (d->bound[is] == BOUND_USERDEF) {
       rc = userdef_side(d, is, stage, v, b);
       if (rc) {

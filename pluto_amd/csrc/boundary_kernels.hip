@@ -50,8 +50,16 @@ struct FillSide {
   int nop, dir, end_side, kind;   // kind: 0 outflow, 1 periodic, 2 reflective
 };
 
-__global__ void __launch_bounds__(256) k_bound_fill(GhostBox b, FillSide f)
+// one side, or both sides of an axis (blockIdx.z): neither reads a cell that
+// the other writes (a box has as many interior cells as ghost zones)
+struct FillSides {
+  FillSide side[2];
+};
+
+__global__ void __launch_bounds__(256) k_bound_fill(GhostBox b, FillSides fs)
 {
+  const FillSide& f = fs.side[blockIdx.z];
+  if ((int)blockIdx.y >= f.nop) return;
   const FillOp& o = f.op[blockIdx.y];
   const int d = f.dir, ta = d == 0 ? 1 : 0, tb = d == 2 ? 1 : 2;
   const int na = o.hi[ta] - o.lo[ta] + 1, nb = o.hi[tb] - o.lo[tb] + 1;
@@ -81,8 +89,13 @@ struct DivbSide {
   int dir, end_side;
 };
 
-__global__ void __launch_bounds__(256) k_bound_divb(GhostBox b, DivbSide f)
+struct DivbSides {
+  DivbSide side[2];
+};
+
+__global__ void __launch_bounds__(256) k_bound_divb(GhostBox b, DivbSides fs)
 {
+  const DivbSide& f = fs.side[blockIdx.y];
   const int d = f.dir, ta = d == 0 ? 1 : 0, tb = d == 2 ? 1 : 2;
   const int na = b.t[ta], nb = b.t[tb];
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -151,8 +164,8 @@ void flip_sign(int dir, int type, double sgn[8])
 
 // FillMagneticField on side (d, end_side) and, with bc set, the
 // cell-centred normal field of CT_AverageNormalMagField
-static int launch_divb_side(const GhostBox& b, int d, int end_side, double* bc, double* const* vs,
-                            const double* const* area, const double* area_c, hipStream_t s)
+static DivbSide divb_side(int d, int end_side, double* bc, double* const* vs,
+                          const double* const* area, const double* area_c)
 {
   DivbSide g{};
   for (int a = 0; a < 3; a++) {
@@ -160,22 +173,27 @@ static int launch_divb_side(const GhostBox& b, int d, int end_side, double* bc, 
     g.area[a] = area ? area[a] : nullptr;
     g.area_c[a] = area_c ? area_c[a] : 0.0;
   }
-  if (!area && !area_c) return (int)hipErrorInvalidValue;
   g.bc = bc;
   g.dir = d;
   g.end_side = end_side;
+  return g;
+}
+
+static int launch_divb(const GhostBox& b, const DivbSides& g, int sides, hipStream_t s)
+{
+  const int d = g.side[0].dir;
   const long lines = (long)b.t[d == 0 ? 1 : 0] * b.t[d == 2 ? 1 : 2];
-  hipLaunchKernelGGL(k_bound_divb, dim3((unsigned)((lines + 255) / 256)), dim3(256), 0, s, b, g);
+  hipLaunchKernelGGL(k_bound_divb, dim3((unsigned)((lines + 255) / 256), sides), dim3(256), 0, s, b, g);
   return (int)hipGetLastError();
 }
 
-int launch_boundary_side(const GhostBox& b, int side, int type, double* const* vc,
-                         double* const* vs, const double* const* area, const double* area_c,
-                         hipStream_t s)
+// the copies of one side; the transverse points of its largest box into most
+static int fill_side(const GhostBox& b, int side, int type, double* const* vc, double* const* vs,
+                     FillSide& f, long& most)
 {
   if (side < 0 || side > 5) return (int)hipErrorInvalidValue;
   const int d = side / 2, end_side = side & 1;
-  FillSide f{};
+  f = FillSide{};
   f.dir = d;
   f.end_side = end_side;
   if (type == BOUND_OUTFLOW) f.kind = 0;
@@ -193,7 +211,6 @@ int launch_boundary_side(const GhostBox& b, int side, int type, double* const* v
   }
   lo[d] = end_side ? b.end[d] + 1 : b.beg[d] - 1;
   hi[d] = end_side ? b.t[d] - 1 : 0;
-  long most = 0;
   auto add = [&](double* p, int ext, const int* l, const int* h, double sg) {
     FillOp& o = f.op[f.nop++];
     o.p = p;
@@ -218,12 +235,45 @@ int launch_boundary_side(const GhostBox& b, int side, int type, double* const* v
     else h[a] -= 1;
     add(vs[a], a, l, h, sgn[kBX1 + a]);
   }
-  const dim3 bl(256);
-  hipLaunchKernelGGL(k_bound_fill, dim3((unsigned)((most + 255) / 256), f.nop), bl, 0, s, b, f);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || f.kind == 1) return (int)e;
-  return launch_divb_side(b, d, end_side, f.kind == 0 ? vc[kBX1 + d] : nullptr, vs, area, area_c,
-                          s);
+  return 0;
+}
+
+static int launch_sides(const GhostBox& b, int first, const int* type, int sides, double* const* vc,
+                        double* const* vs, const double* const* area, const double* area_c,
+                        hipStream_t s)
+{
+  FillSides f{};
+  DivbSides g{};
+  long most = 0;
+  int nop = 0, nd = 0;
+  for (int q = 0; q < sides; q++) {
+    const int rc = fill_side(b, first + q, type[q], vc, vs, f.side[q], most);
+    if (rc) return rc;
+    nop = f.side[q].nop > nop ? f.side[q].nop : nop;
+    if (f.side[q].kind == 1) continue;
+    if (!area && !area_c) return (int)hipErrorInvalidValue;
+    const int d = (first + q) / 2;
+    g.side[nd++] = divb_side(d, (first + q) & 1, f.side[q].kind == 0 ? vc[kBX1 + d] : nullptr, vs, area,
+                             area_c);
+  }
+  hipLaunchKernelGGL(k_bound_fill, dim3((unsigned)((most + 255) / 256), nop, sides), dim3(256), 0, s, b, f);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess || !nd ? (int)e : launch_divb(b, g, nd, s);
+}
+
+int launch_boundary_side(const GhostBox& b, int side, int type, double* const* vc,
+                         double* const* vs, const double* const* area, const double* area_c,
+                         hipStream_t s)
+{
+  return launch_sides(b, side, &type, 1, vc, vs, area, area_c, s);
+}
+
+int launch_boundary_axis(const GhostBox& b, int axis, const int type[2], double* const* vc,
+                         double* const* vs, const double* const* area, const double* area_c,
+                         hipStream_t s)
+{
+  if (axis < 0 || axis > 2) return (int)hipErrorInvalidValue;
+  return launch_sides(b, 2 * axis, type, 2, vc, vs, area, area_c, s);
 }
 
 int launch_boundary_fill_normal(const GhostBox& b, int side, double* const* vc, double* const* vs,
@@ -231,7 +281,10 @@ int launch_boundary_fill_normal(const GhostBox& b, int side, double* const* vc, 
 {
   if (side < 0 || side > 5) return (int)hipErrorInvalidValue;
   const int d = side / 2;
-  return launch_divb_side(b, d, side & 1, vc[kBX1 + d], vs, area, area_c, s);
+  if (!area && !area_c) return (int)hipErrorInvalidValue;
+  DivbSides g{};
+  g.side[0] = divb_side(d, side & 1, vc[kBX1 + d], vs, area, area_c);
+  return launch_divb(b, g, 1, s);
 }
 
 }  // namespace pgpu
