@@ -431,35 +431,25 @@ extern "C" int pgpu_set_state(pgpu_domain* d, const double* prim, const double* 
 extern "C" int pgpu_get_state(pgpu_domain* d, double* prim, double* bx, double* by, double* bz)
 {
   if (!d) return fail(PGPU_EINVAL, "domain is NULL");
-  if (d->g.ghost) {
-    // the interior cells and their upper faces
-    const GhostBox& b = d->gb;
-    const long ni = (long)b.n[0] * b.n[1] * b.n[2];
-    std::vector<double> big((size_t)d->g.n);
-    double* faces[3] = {bx, by, bz};
-    for (int q = 0; q < 11; q++) {
-      double* dst = q < 8 ? (prim ? prim + (size_t)q * ni : nullptr) : faces[q - 8];
-      if (!dst) continue;
-      HIP_TRY(hipMemcpyAsync(big.data(), q < 8 ? d->V[q] : d->bA[q - 8],
-                             (size_t)d->g.n * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-      HIP_TRY(hipStreamSynchronize(d->stream));
-      for (int k = 0; k < b.n[2]; k++)
-        for (int j = 0; j < b.n[1]; j++)
-          for (int i = 0; i < b.n[0]; i++)
-            dst[((long)k * b.n[1] + j) * b.n[0] + i] = big[gh_index(b, i, j, k)];
-    }
-    return PGPU_OK;
-  }
   const Geo& g = d->g;
-  const size_t nb = (size_t)g.n * sizeof(double);
-  if (prim)
-    for (int q = 0; q < 8; q++)
-      HIP_TRY(hipMemcpyAsync(prim + (size_t)q * g.n, d->V[q], nb, hipMemcpyDeviceToHost, d->stream));
+  ReadSrc src;
+  const GhostBox& b = d->gb;
+  const int n[3] = {g.ghost ? b.n[0] : g.nx, g.ghost ? b.n[1] : g.ny, g.ghost ? b.n[2] : g.nz};
+  for (int a = 0; a < 3; a++) src.n[a] = n[a];
+  src.row = g.nx;
+  src.plane = (long)g.nx * g.ny;
+  src.first = g.ghost ? gh_index(b, 0, 0, 0) : 0;   // a ghosted box: the interior cells, their upper faces
+  const long ni = (long)n[0] * n[1] * n[2];
   double* faces[3] = {bx, by, bz};
-  for (int a = 0; a < 3; a++)
-    if (faces[a])
-      HIP_TRY(hipMemcpyAsync(faces[a], d->bA[a], nb, hipMemcpyDeviceToHost, d->stream));
-  HIP_TRY(hipStreamSynchronize(d->stream));
+  double* dst[11];
+  for (int q = 0; q < 11; q++) {
+    double* to = q < 8 ? (prim ? prim + (size_t)q * ni : nullptr) : faces[q - 8];
+    if (!to) continue;
+    src.a[src.na] = q < 8 ? d->V[q] : d->bA[q - 8];
+    dst[src.na++] = to;
+  }
+  const int rc = readback(d->rb, src, dst, d->stream);
+  if (rc) return fail(PGPU_EDEVICE, "state download failed: %s", hipGetErrorString((hipError_t)rc));
   return PGPU_OK;
 }
 

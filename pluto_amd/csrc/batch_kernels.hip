@@ -445,6 +445,7 @@ struct pgpu_batch {
   };
   std::vector<Branch> br;
   int nbr = 0;                   // branches of the captured step
+  Readback rb;                   // staging of pgpu_batch_get_patch
 };
 
 // one stage of a stack through the fused kernels
@@ -834,18 +835,23 @@ extern "C" int pgpu_batch_get_patch(pgpu_batch* b, int p, double* prim, double* 
                                     double* bz)
 {
   if (!patch_ok(b, p)) return fail(PGPU_EINVAL, "bad patch index");
-  if (hipStreamSynchronize(b->stream) != hipSuccess) return fail(PGPU_EDEVICE, "stream synchronisation failed");
   const int n = b->edge[p];
-  const size_t nz = (size_t)n * n * n, nb = nz * sizeof(double);
+  const size_t nz = (size_t)n * n * n;
   const long o = b->off[p];
-  hipError_t err = hipSuccess;
-  if (prim)
-    for (int q = 0; q < 8 && err == hipSuccess; q++)
-      err = hipMemcpy(prim + (size_t)q * nz, b->A.V[q] + o, nb, hipMemcpyDeviceToHost);
+  ReadSrc src;
+  for (int a = 0; a < 3; a++) src.n[a] = n;
+  src.row = n;
+  src.plane = (long)n * n;
   double* f[3] = {bx, by, bz};
-  for (int a = 0; a < 3 && err == hipSuccess; a++)
-    if (f[a]) err = hipMemcpy(f[a], b->A.bA[a] + o, nb, hipMemcpyDeviceToHost);
-  if (err != hipSuccess) return fail(PGPU_EDEVICE, "patch download failed: %s", hipGetErrorString(err));
+  double* dst[11];
+  for (int q = 0; q < 11; q++) {
+    double* to = q < 8 ? (prim ? prim + (size_t)q * nz : nullptr) : f[q - 8];
+    if (!to) continue;
+    src.a[src.na] = (q < 8 ? b->A.V[q] : b->A.bA[q - 8]) + o;
+    dst[src.na++] = to;
+  }
+  const int rc = readback(b->rb, src, dst, b->stream);
+  if (rc) return fail(PGPU_EDEVICE, "patch download failed: %s", hipGetErrorString((hipError_t)rc));
   return PGPU_OK;
 }
 

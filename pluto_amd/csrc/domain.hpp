@@ -7,6 +7,7 @@
 
 #include "../../include/pluto_amd.h"
 #include "boundary_kernels.hpp"
+#include "readback.hpp"
 #include "stage_kernels.hpp"
 
 namespace pgpu {
@@ -117,6 +118,7 @@ struct pgpu_domain {
   pgpu_userdef_fn userdef = nullptr;
   void* userdef_ctx = nullptr;
   std::vector<double> slab_buf;
+  pgpu::Readback rb;   // staging of pgpu_get_state
 };
 
 // Makes a domain of (t[0]+1) x (t[1]+1) x (t[2]+1) cells hold PLUTO's

@@ -1,0 +1,167 @@
+// Read-back of state arrays into the caller's (pageable) memory.
+//
+// A kernel gathers the wanted cells of all arrays straight into pinned host
+// buffers over the link, a ring of four buffers ahead of the host threads
+// that copy them out.  hipMemcpy to pageable memory moved 16 GB/s, one copy
+// and one wait per array, and a ghosted box's arrays came whole and were cut
+// on the host by one thread: 128^3 read back from a periodic box 11.3 -> 3.9
+// ms (48 GB/s; the link 57), from a bounded one 20.7 -> 3.9 ms, 32^3 0.27 ->
+// 0.15 and 0.33 -> 0.15 ms, 96 patches of edges 16 to 64 one by one 47 -> 26.
+
+#include "readback.hpp"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <thread>
+#include <vector>
+
+namespace pgpu {
+
+namespace {
+
+// elements e0 .. e0 + n - 1 of the arrays one after another
+__global__ void __launch_bounds__(256) k_gather_cells(ReadSrc s, long e0, long n, double* out)
+{
+  const long ni = (long)s.n[0] * s.n[1] * s.n[2];
+  for (long t = (long)blockIdx.x * 256 + threadIdx.x; t < n; t += (long)gridDim.x * 256) {
+    const long e = e0 + t, q = e / ni;
+    const unsigned c = (unsigned)(e - q * ni);   // (a domain's arrays are under 2^32 cells)
+    const unsigned r = c / (unsigned)s.n[0], i = c - r * (unsigned)s.n[0];
+    const unsigned k = r / (unsigned)s.n[1], j = r - k * (unsigned)s.n[1];
+    out[t] = s.a[q][s.first + (long)k * s.plane + (long)j * s.row + i];
+  }
+}
+
+int make_ring(Readback& rb)
+{
+  if (rb.elems) return 0;
+  for (long el = 1l << 19; el >= 1l << 15; el >>= 2) {   // 4 MiB buffers, less where that is refused
+    hipError_t e = hipSuccess;
+    for (int q = 0; q < Readback::NB && e == hipSuccess; q++) {
+      if (!rb.ev[q]) e = hipEventCreateWithFlags(&rb.ev[q], hipEventDisableTiming);
+      if (e == hipSuccess) e = hipHostMalloc((void**)&rb.h[q], (size_t)el * sizeof(double), hipHostMallocDefault);
+    }
+    if (e == hipSuccess) {
+      rb.elems = el;
+      return 0;
+    }
+    for (int q = 0; q < Readback::NB; q++) {
+      if (rb.h[q]) (void)hipHostFree(rb.h[q]);
+      rb.h[q] = nullptr;
+    }
+    (void)hipGetLastError();
+  }
+  return (int)hipErrorOutOfMemory;
+}
+
+}  // namespace
+
+Readback::~Readback()
+{
+  for (int q = 0; q < NB; q++) {
+    if (h[q]) (void)hipHostFree(h[q]);
+    if (ev[q]) (void)hipEventDestroy(ev[q]);
+  }
+}
+
+int readback(Readback& rb, const ReadSrc& src, double* const* dst, hipStream_t s)
+{
+  constexpr int NB = Readback::NB;
+  const long ni = (long)src.n[0] * src.n[1] * src.n[2], total = ni * src.na;
+  if (total <= 0) return 0;
+  // (the caller's current device may be another)
+  struct OnDevice {
+    int was = -1;
+    explicit OnDevice(hipStream_t s)
+    {
+      int cur = 0, own = 0;
+      if (hipGetDevice(&cur) == hipSuccess && hipStreamGetDevice(s, &own) == hipSuccess && own != cur &&
+          hipSetDevice(own) == hipSuccess)
+        was = cur;
+    }
+    ~OnDevice()
+    {
+      if (was >= 0) (void)hipSetDevice(was);
+    }
+  } on(s);
+  if (const int rc = make_ring(rb)) return rc;
+  const long ch = rb.elems, nch = (total + ch - 1) / ch;
+
+  // elements [e0, e1) of the concatenation, held from h on, to their arrays
+  auto copy_out = [&](const double* h, long e0, long e1) {
+    for (long e = e0; e < e1;) {
+      const long q = e / ni, c = e - q * ni, m = std::min(e1 - e, ni - c);
+      memcpy(dst[q] + c, h + (e - e0), (size_t)m * sizeof(double));
+      e += m;
+    }
+  };
+
+  // chunk c is in its buffer when ready > c; left: threads still copying it
+  std::atomic<long> ready{0};
+  std::atomic<bool> stop{false};
+  std::atomic<int> left[NB];
+  for (auto& l : left) l.store(0);
+  std::atomic<int> nworkers{-1};   // (set before the first chunk is ready)
+  auto work = [&](int w) {
+    for (long c = 0; c < nch; c++) {
+      while (ready.load(std::memory_order_acquire) <= c) {
+        if (stop.load()) return;
+        std::this_thread::yield();
+      }
+      const int nw = nworkers.load();
+      const long e0 = c * ch, len = std::min(ch, total - e0);
+      const long b = len * w / nw, e = len * (w + 1) / nw;
+      copy_out(rb.h[c % NB] + b, e0 + b, e0 + e);
+      left[c % NB].fetch_sub(1, std::memory_order_release);
+    }
+  };
+  // a thread copies about 10 GB/s and starts in about 20 us: from two chunks
+  // on, up to eight
+  std::vector<std::thread> th;
+  const int want = nch < 2 ? 0 : (int)std::min(8u, std::max(1u, std::thread::hardware_concurrency() / 2));
+  try {
+    th.reserve(want);
+    for (int w = 0; w < want; w++) th.emplace_back(work, w);
+  } catch (...) {   // fewer threads, or none: this one copies
+  }
+  const int nw = (int)th.size();
+  nworkers.store(nw);
+
+  hipError_t err = hipSuccess;
+  long issued = 0, got = 0;
+  while (got < nch && err == hipSuccess) {
+    while (issued < nch && issued - got < NB && left[issued % NB].load(std::memory_order_acquire) == 0) {
+      const long e0 = issued * ch, len = std::min(ch, total - e0);
+      const long nwg = (len + 1023) / 1024;
+      left[issued % NB].store(nw);
+      hipLaunchKernelGGL(k_gather_cells, dim3((unsigned)nwg), dim3(256), 0, s, src, e0, len, rb.h[issued % NB]);
+      err = hipGetLastError();
+      if (err == hipSuccess) err = hipEventRecord(rb.ev[issued % NB], s);
+      if (err != hipSuccess) break;
+      issued++;
+    }
+    if (err != hipSuccess) break;
+    if (issued == got) {   // every buffer is still being copied out
+      std::this_thread::yield();
+      continue;
+    }
+    err = hipEventSynchronize(rb.ev[got % NB]);
+    if (err != hipSuccess) break;
+    if (nw == 0) {
+      const long e0 = got * ch;
+      copy_out(rb.h[got % NB], e0, std::min(e0 + ch, total));
+      left[got % NB].store(0);
+    }
+    ready.store(++got, std::memory_order_release);
+  }
+  // (only a failure stops the threads: after the last chunk they still copy)
+  if (err != hipSuccess) {
+    stop.store(true);
+    (void)hipStreamSynchronize(s);   // nothing writes the buffers any more
+  }
+  for (auto& x : th) x.join();
+  return (int)err;
+}
+
+}  // namespace pgpu

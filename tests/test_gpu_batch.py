@@ -208,6 +208,7 @@ def test_batch_branches(native, edges):
     """Stacks on one branch and on four, with patches of the persistent
     kernel beside them: several runs with reads between them equal the
     persistent mode's single run."""
+    from pluto_amd import problems as P
     _say("case: batch branches %s" % edges)
     states = [P.random_mhd_3d(n, seed=700 + p) for p, n in enumerate(edges)]
     a, b = native.Batch(edges), native.Batch(edges)

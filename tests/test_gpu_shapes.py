@@ -89,3 +89,26 @@ def test_emf_tiles(shape, kind):
         check(shape, dims=2 if shape[0] == 1 else 3)
     finally:
         native.set_emf_kernel()
+
+
+# read-back: less than one staging buffer (2^19 values), just over one and
+# several with a cut last one, interior of a bounded box, single arrays
+@pytest.mark.parametrize("shape", [(3, 4, 5), (36, 37, 36), (47, 50, 49), (90, 81, 77)])
+@pytest.mark.parametrize("bounded", [False, True])
+def test_readback(shape, bounded):
+    import ctypes
+
+    import numpy as np
+
+    from pluto_amd import native
+    st = box_state(shape)
+    dom = native.Domain(st.shape, 3, st.spacing(), bounds=["periodic"] * 6 if bounded else None)
+    dom.set_state(st)
+    for _ in range(20):
+        out = dom.get_state(st)
+        assert_states_equal(out, st, "%s bounded %s" % (shape, bounded))
+    one = np.full(shape, -1.0)
+    native.check(native.lib().pgpu_get_state(dom.h, None, None, one.ctypes.data_as(
+        ctypes.POINTER(ctypes.c_double)), None))
+    assert np.array_equal(one, st.by)
+    dom.close()
