@@ -115,6 +115,125 @@ __global__ void __launch_bounds__(256) k_emf_faces(Geo g, StageIn in, Sweeps sw,
   emf_faces_cell<MODE>(g, p, in, sw, e);
 }
 
+// UCT0 and UCT_CONTACT in 3D, marching up z: a workgroup takes 256 consecutive columns of
+// the plane and kz planes.  What Ex and Ey of plane k read from plane k+1 (the
+// cell EMFs of three columns, four face values) is computed once, kept in
+// registers and is plane k's own part at the next step, so a cell reads about
+// 47 values (UCT_CONTACT) where the per-cell form reads over a hundred and
+// forms every cell EMF up to eight times.  Same expressions in the same
+// order.  UCT_CONTACT 256^3 1184 -> 644 us a launch, 128^3 137 -> 91, 131 x 93
+// x 77 75 -> 38; UCT0 607 -> 544, 83 -> 77, 38 -> 33.  (ARITHMETIC, which reads
+// no cell EMF, is bound by its 12 values in either form: 228 us per cell, 237
+// marching.)
+template <int MODE>
+__global__ void __launch_bounds__(256) k_emf_faces_z(Geo g, StageIn in, Sweeps sw, EdgeOut e, int kz)
+{
+  const unsigned col = blockIdx.x * 256u + threadIdx.x;
+  const unsigned nxy = (unsigned)g.nx * (unsigned)g.ny;
+  if (col >= nxy) return;
+  const int j = (int)(col / (unsigned)g.nx), i = (int)(col - (unsigned)j * (unsigned)g.nx);
+  // byte offsets in a plane: the cell, and those one further along x, y, both
+  const unsigned jp = (unsigned)wrap2(j, 1, g.ny) * (unsigned)g.nx, ip = (unsigned)wrap2(i, 1, g.nx);
+  const unsigned o00 = col * 8u, o10 = ((unsigned)j * (unsigned)g.nx + ip) * 8u, o01 = (jp + (unsigned)i) * 8u,
+                 o11 = (jp + ip) * 8u;
+  const int k0 = blockIdx.y * kz, k1 = min(k0 + kz, g.nz);
+  // component A of the cell EMF at byte offset o of the arrays
+  auto E = [&](int A, unsigned o) -> double {
+    if (A == 0) return at_byte(in.V[VX3], o) * at_byte(in.V[BX2], o) - at_byte(in.V[VX2], o) * at_byte(in.V[BX3], o);
+    if (A == 1) return at_byte(in.V[VX1], o) * at_byte(in.V[BX3], o) - at_byte(in.V[VX3], o) * at_byte(in.V[BX1], o);
+    return at_byte(in.V[VX2], o) * at_byte(in.V[BX1], o) - at_byte(in.V[VX1], o) * at_byte(in.V[BX2], o);
+  };
+  // upwind sign of the mass flux at the d-face at byte offset o (ct_emf.c:136-141)
+  auto S = [&](int d, unsigned o) -> int {
+    const double f = at_byte(sw.d[d].dv[0], o);
+    return f > 1.e-6 ? 1 : (f < -1.e-6 ? -1 : 0);
+  };
+  // what plane k + 1 gives to the edges of plane k
+  struct Roll {
+    double ex00, ex01, ey00, ey10;   // cell EMFs
+    double eyi, exj;                 // face EMFs of the x and y faces
+    int sx = 0, sy = 0;              // mass flux signs there
+  };
+  auto roll = [&](unsigned pk) {
+    Roll r;
+    r.ex00 = E(0, pk + o00);
+    r.ex01 = E(0, pk + o01);
+    r.ey00 = E(1, pk + o00);
+    r.ey10 = E(1, pk + o10);
+    r.eyi = at_byte(sw.d[0].SR, pk + o00);
+    r.exj = at_byte(sw.d[1].SR, pk + o00);
+    if constexpr (MODE == EMF_UCT_CONTACT) {
+      r.sx = S(0, pk + o00);
+      r.sy = S(1, pk + o00);
+    }
+    return r;
+  };
+  Roll c = roll((unsigned)k0 * nxy * 8u);
+  for (int k = k0; k < k1; k++) {
+    const unsigned pk = (unsigned)k * nxy * 8u;
+    const Roll n = roll((unsigned)wrap2(k, 1, g.nz) * nxy * 8u);
+    const double ezi00 = at_byte(sw.d[0].SL, pk + o00), ezi01 = at_byte(sw.d[0].SL, pk + o01);
+    const double ezj00 = at_byte(sw.d[1].SL, pk + o00), ezj10 = at_byte(sw.d[1].SL, pk + o10);
+    const double eyk00 = at_byte(sw.d[2].SL, pk + o00), eyk10 = at_byte(sw.d[2].SL, pk + o10);
+    const double exk00 = at_byte(sw.d[2].SR, pk + o00), exk01 = at_byte(sw.d[2].SR, pk + o01);
+    double ez, ex, ey;
+    if constexpr (MODE == EMF_UCT0) {
+      // ct_emf.c:261-283: each face EMF doubled minus the mean of its two cells'
+      auto U0 = [](double f, double a, double b) { return f * 2.0 - 0.5 * (a + b); };
+      const double z00 = E(2, pk + o00), z10 = E(2, pk + o10), z01 = E(2, pk + o01), z11 = E(2, pk + o11);
+      ez = 0.25 * (U0(ezi00, z00, z10) + U0(ezi01, z01, z11) + U0(ezj00, z00, z01) + U0(ezj10, z10, z11));
+      ex = 0.25 * (U0(exk00, c.ex00, n.ex00) + U0(exk01, c.ex01, n.ex01) + U0(c.exj, c.ex00, c.ex01) +
+                   U0(n.exj, n.ex00, n.ex01));
+      ey = 0.25 * (U0(c.eyi, c.ey00, c.ey10) + U0(n.eyi, n.ey00, n.ey10) + U0(eyk00, c.ey00, n.ey00) +
+                   U0(eyk10, c.ey10, n.ey10));
+    } else {
+      ez = ezi00 + ezi01 + ezj00 + ezj10;
+      ex = exk00 + exk01 + c.exj + n.exj;
+      ey = c.eyi + n.eyi + eyk00 + eyk10;
+      // the term of the upwind side, or the mean of both (s == 0)
+      auto up = [](int s, double a, double b) { return s == 0 ? 0.5 * (a + b) : (s > 0 ? a : b); };
+      const double z00 = E(2, pk + o00), z10 = E(2, pk + o10), z01 = E(2, pk + o01), z11 = E(2, pk + o11);
+      const int sz = S(2, pk + o00);
+      ez += up(c.sx, ezj00 - z00, ezj10 - z10);
+      ez += up(c.sy, ezi00 - z00, ezi01 - z01);
+      ez -= up(S(1, pk + o10), z10 - ezi00, z11 - ezi01);
+      ez -= up(S(0, pk + o01), z01 - ezj00, z11 - ezj10);
+      ez *= 0.25;
+      ex += up(c.sy, exk00 - c.ex00, exk01 - c.ex01);
+      ex += up(sz, c.exj - c.ex00, n.exj - n.ex00);
+      ex -= up(S(2, pk + o01), c.ex01 - c.exj, n.ex01 - n.exj);
+      ex -= up(n.sy, n.ex00 - exk00, n.ex01 - exk01);
+      ex *= 0.25;
+      ey += up(c.sx, eyk00 - c.ey00, eyk10 - c.ey10);
+      ey += up(sz, c.eyi - c.ey00, n.eyi - n.ey00);
+      ey -= up(S(2, pk + o10), c.ey10 - c.eyi, n.ey10 - n.eyi);
+      ey -= up(n.sx, n.ey00 - eyk00, n.ey10 - eyk10);
+      ey *= 0.25;
+    }
+    at_byte(e.ez, pk + o00) = ez;
+    at_byte(e.ex, pk + o00) = ex;
+    at_byte(e.ey, pk + o00) = ey;
+    c = n;
+  }
+}
+
+template <int MODE>
+static void launch_emf_faces(const Geo& g, const StageIn& in, const Sweeps& sw, const EdgeOut& e,
+                             hipStream_t s)
+{
+  if (g.dims == 3 && (unsigned long long)g.n * 8ull < (1ull << 32)) {   // 32-bit byte offsets
+    // 16 planes a segment (each segment reads one plane twice), fewer where
+    // that would leave less than eight workgroups a CU
+    const unsigned wgs = (unsigned)(((long)g.nx * g.ny + 255) / 256);
+    int kz = 16;
+    while (kz > 1 && (long)wgs * ((g.nz + kz - 1) / kz) < 2048) kz /= 2;
+    hipLaunchKernelGGL(k_emf_faces_z<MODE>, dim3(wgs, (g.nz + kz - 1) / kz), dim3(256), 0, s, g, in, sw, e, kz);
+  } else {
+    hipLaunchKernelGGL(k_emf_faces<MODE>, dim3((g.nx + 63) / 64, (g.ny + 3) / 4, g.nz), dim3(64, 4), 0, s, g, in,
+                       sw, e);
+  }
+}
+
 // z-marching EMF (3D): a workgroup covers a bx x by patch of a plane and
 // marches kz planes.  The stencil reads 100 values per cell; 26 of them
 // (field, i-offset, j-offset) are read on both planes k and k+1, and the
@@ -390,9 +509,13 @@ static bool enqueue_emf(const Geo& g, const StageIn& in, const Sweeps& sw, const
   if (g.emf_avg == EMF_ARITHMETIC) {
     PGPU_TIMED(KT_EMF, k_emf_faces<EMF_ARITHMETIC>, grid_of(g), kBlock, 0, s, g, in, sw, e);
   } else if (g.emf_avg == EMF_UCT0) {
-    PGPU_TIMED(KT_EMF, k_emf_faces<EMF_UCT0>, grid_of(g), kBlock, 0, s, g, in, sw, e);
+    if (kt) kt->begin(KT_EMF, s);
+    launch_emf_faces<EMF_UCT0>(g, in, sw, e, s);
+    if (kt) kt->end(KT_EMF, s);
   } else if (g.emf_avg == EMF_UCT_CONTACT) {
-    PGPU_TIMED(KT_EMF, k_emf_faces<EMF_UCT_CONTACT>, grid_of(g), kBlock, 0, s, g, in, sw, e);
+    if (kt) kt->begin(KT_EMF, s);
+    launch_emf_faces<EMF_UCT_CONTACT>(g, in, sw, e, s);
+    if (kt) kt->end(KT_EMF, s);
   } else if ((g_emf_kernel || g.pz > 0 || g.dims != 3) &&
              launch_emf_lds(g, in, sw, e, s, g_emf_kernel ? g_emf_kernel : 3, g_emf_lds_kz, kt,
                             f32_state ? 2 : (f32_faces ? 1 : 0))) {

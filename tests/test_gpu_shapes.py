@@ -36,18 +36,18 @@ def box_state(shape, dims=3, seed=11):
     return P.assemble(1.0 + 0.3 * field(), v, 1.0 + 0.3 * field(), *b, dims, (1.0, 1.0, 1.0))
 
 
-def check(shape, steps=2, dims=3, **kw):
+def check(shape, steps=2, dims=3, emf="uct_hll", **kw):
     from pluto_amd import native
     st = box_state(shape, dims)
     dt = 0.05 / max(shape)
-    dom = native.Domain.from_state(st, **kw)
+    dom = native.Domain.from_state(st, emf_average=emf, **kw)
     dom.set_dt(dt)
     dom.run(steps)
     dom.sync()
     out = dom.get_state(st)
     dom.close()
     ref = st.copy()
-    O.run(ref, steps, dt)
+    O.run(ref, steps, dt, emf=emf)
     assert_states_equal(out, ref, "%s" % (shape,))
 
 
@@ -89,6 +89,16 @@ def test_emf_tiles(shape, kind):
         check(shape, dims=2 if shape[0] == 1 else 3)
     finally:
         native.set_emf_kernel()
+
+
+# the face EMF averages marching up z: planes of less than one workgroup, one
+# and several with a cut last one, segments of 1 plane, 2 with a remainder and
+# 16 with a remainder; 2D (per cell)
+@pytest.mark.parametrize("shape", [(3, 3, 3), (5, 16, 16), (7, 86, 3), (9, 17, 31), (33, 130, 130),
+                                   (37, 181, 200), (19, 600, 450), (1, 9, 32)])
+@pytest.mark.parametrize("emf", ["uct0", "uct_contact", "arithmetic"])
+def test_emf_faces(shape, emf):
+    check(shape, dims=2 if shape[0] == 1 else 3, emf=emf)
 
 
 # read-back: less than one staging buffer (2^19 values), just over one and
