@@ -652,22 +652,11 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
     const R bfy = kPrefetch ? bfy_n : R(at_byte(in.b[1], c));
 
     // x reconstruction of cell (i, j)
-    double u[5];
     R vmx[NV];
     {
       R w0[NV], a[NV], b[NV], vpx[NV];
 #pragma unroll
       for (int q = 0; q < NV; q++) w0[q] = rv(s0, q, t);
-      if (STAGE == 1) {   // U0 from the FP64 state
-        double v[NV];
-#pragma unroll
-        for (int q = 0; q < NV; q++) v[q] = double(ring[(s0 * NV + q) * nt + t]);
-        u[0] = v[RHO];
-        u[1] = v[RHO] * v[VX1];
-        u[2] = v[RHO] * v[VX2];
-        u[3] = v[RHO] * v[VX3];
-        u[4] = total_energy(v, g.gmm1);
-      }
 #pragma unroll
       for (int q = 0; q < XROW_NV; q++) {
         a[xrow_var(q)] = rv(s0, xrow_var(q), tl);
@@ -692,7 +681,7 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
     }
 
     // x interface i-1/2
-    R fxl[6], cmxl, xsl, xsr, xe[3];
+    R xsl, xsr, xe[3];
     {
       R vL[NV], vR[NV];
 #pragma unroll
@@ -704,9 +693,7 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
       vR[BX1] = bface;
       RiemannOut<R> r;
       riemann<S, 0, E == FACE_BFLUX>(vL, vR, gam, gm1, r, g.dims == 2);
-      fxl[0] = r.f[RHO]; fxl[1] = r.f[VX1]; fxl[2] = r.f[VX2];
-      fxl[3] = r.f[VX3]; fxl[4] = r.f[ENG]; fxl[5] = r.press;
-      cmxl = r.cmax;
+      const R fxl[6] = {r.f[RHO], r.f[VX1], r.f[VX2], r.f[VX3], r.f[ENG], r.press};
       if constexpr (E == FACE_BFLUX) {
         xe[0] = -r.f[BX2];   // ezi, eyi (ct_emf.c:131-133)
         xe[1] = r.f[BX3];
@@ -717,7 +704,7 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
       }
 #pragma unroll
       for (int q = 0; q < 6; q++) xf[q * nt + t] = fxl[q];
-      xf[6 * nt + t] = cmxl;
+      xf[6 * nt + t] = r.cmax;
       if (act) {
         const double rm = double(r.mach);
         if (in_sweep(g, 0, ic - 1, j, k)) mach = rm > mach ? rm : mach;
@@ -740,12 +727,6 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
         fstore(fd.SR[0], cf, xsr);
       }
     }
-    double rx[5], cdt = 0.0;
-#pragma unroll
-    for (int q = 0; q < 5; q++) rx[q] = -dtdx * (double(xf[q * nt + tr]) - double(fxl[q]));
-    rx[1] -= dtdx * (double(xf[5 * nt + tr]) - double(fxl[5]));
-    if (STAGE == 1) cdt += 0.5 * (double(cmxl) + double(xf[6 * nt + tr])) * g.inv_dx[0];
-
     // y reconstruction of cell (i, j+1) and the y interface j+1/2
     R vpn[NV], vmn[NV];
     {
@@ -786,13 +767,34 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
         }
         const double rm = double(r.mach);
         if (in_sweep(g, 1, ic, j, k)) mach = rm > mach ? rm : mach;
+        // the x fluxes and signal speeds of both faces, still in LDS: held in
+        // registers through the y solve they and U0 spilled (256^3, us a
+        // launch: Roe 2012 -> 1390, HLLD with magnetic face fluxes 1385 ->
+        // 1225; HLLD alone fitted before too, 1186 either way)
+        double rx[5], cdt = 0.0;
+#pragma unroll
+        for (int q = 0; q < 5; q++) rx[q] = -dtdx * (double(xf[q * nt + tr]) - double(xf[q * nt + t]));
+        rx[1] -= dtdx * (double(xf[5 * nt + tr]) - double(xf[5 * nt + t]));
+        if (STAGE == 1) cdt += 0.5 * (double(xf[6 * nt + t]) + double(xf[6 * nt + tr])) * g.inv_dx[0];
         double ry[5];
 #pragma unroll
         for (int q = 0; q < 5; q++) ry[q] = -dtdy * (double(fcur[q]) - double(fyb[q]));
         ry[2] -= dtdy * (double(fcur[5]) - double(fyb[5]));
+        double u[5];
         if (STAGE == 2) {
 #pragma unroll
           for (int q = 0; q < 5; q++) u[q] = U0[q];
+        } else {
+          // U0 from the FP64 state of row j, still in the ring (formed before
+          // the solves it held ten registers through both of them)
+          double v[NV];
+#pragma unroll
+          for (int q = 0; q < NV; q++) v[q] = double(ring[(s0 * NV + q) * nt + t]);
+          u[0] = v[RHO];
+          u[1] = v[RHO] * v[VX1];
+          u[2] = v[RHO] * v[VX2];
+          u[3] = v[RHO] * v[VX3];
+          u[4] = total_energy(v, g.gmm1);
         }
 #pragma unroll
         for (int q = 0; q < 5; q++) u[q] += rx[q];
