@@ -25,6 +25,7 @@
 #include "fused_kernels.hpp"
 #include "mhd_adjoint.hpp"
 #include "mhd_device.hpp"
+#include "stage_cells.hpp"
 #include "stage_kernels.hpp"
 
 namespace pgpu {
@@ -86,7 +87,7 @@ struct AdjArrays {
   double* lamBc[3];     // adjoint of the cell-centred field (temporary)
   double* VN[8];        // forward V^{n+1}
   double* bN[3];        // forward b^{n+1}
-  double* ep[3][28];    // per-edge partials of the EMF adjoint, per edge family
+  double* ep[3][12];    // per-edge partials of the EMF adjoint, per edge family
   double* sw1[3][5];    // stage-1 sweep outputs kept for its reverse: SR, SL, dv[3]
 };
 
@@ -154,62 +155,89 @@ k_adj_ct(Geo g, AdjArrays A, const DevScalars* sc)
 // ---------------------------------------------------------------------
 // EMF adjoint in two passes without atomics, for the UCT_HLL edge families
 // with axes (P, Q): Ez = <0,1>, Ex = <1,2>, Ey = <2,0> (the stencils of
-// k_emf).  Pass 1 (per edge, for each family F) stores 28 partials:
-//   0-7   speed adjoints: 0 SP.SR, 2 SP.SL, 4 SQ.SR, 6 SQ.SL, each going to
-//         the cell the edge's max() selected (c or c+Q for SP, c or c+P
-//         for SQ); the gather redoes the comparison, so slots 1, 3, 5, 7
-//         are not stored
-//   8-15  corner products (aq, ap) of SW (c), SE (c+P), NE (c+P+Q), NW (c+Q)
-//   16-27 limited-face contributions: S to c, c+Q, c-Q; N to c+Q, c+2Q, c;
-//         W to c, c+P, c-P; E to c+P, c+2P, c
-// Pass 2 (per cell) gathers what the neighbouring edges sent to the cell.
+// k_emf).  Pass 1 (per edge, for each family F) stores 12 partials:
+//   0-3   speed adjoints SP.SR, SP.SL, SQ.SR, SQ.SL, each going to the cell
+//         the edge's max() selected (c or c+Q for SP, c or c+P for SQ); the
+//         gather redoes the comparison
+//   4-7   adjoints of the corner EMFs of SW (c), SE (c+P), NE (c+P+Q),
+//         NW (c+Q)
+//   8-11  adjoints of the limited faces S, N, W, E
+// Pass 2 (per cell) gathers what the neighbouring edges sent to the cell: it
+// forms the face states and the limiters' branches of the few cells that it
+// needs from the fields, and multiplies there what pass 1 otherwise had to
+// multiply out and store (24 partials an edge).  Both passes are bound by
+// memory, 480 and 580 B a cell instead of 770 and 840: at 128^3 577 -> 318 and
+// 441 -> 369 us a launch.
 // ---------------------------------------------------------------------
 
+// byte offsets of a cell and, periodic, of its neighbours up to two away (32
+// bits: the adjoint's arrays of a box with fields of 4 GiB would not fit the
+// device); one VGPR an address where 64-bit ones took two and a multiply
+struct AdjOffs {
+  unsigned c;
+  unsigned d[3][5];   // [axis][offset + 2], to add to c
+};
+
+__device__ __forceinline__ AdjOffs adj_offs(const Geo& g, const AdjCell& p)
+{
+  AdjOffs o;
+  o.c = (unsigned)p.c * 8u;
+  const unsigned st[3] = {8u, 8u * (unsigned)g.nx, 8u * (unsigned)g.nx * (unsigned)g.ny};
+  const int q[3] = {p.i, p.j, p.k}, n[3] = {g.nx, g.ny, g.nz};
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int m = -2; m <= 2; m++) {
+      const int w = wrap2(q[a], m, n[a]) - q[a];
+      o.d[a][m + 2] = m == 0 ? 0u : (unsigned)w * st[a];
+    }
+  return o;
+}
+
 template <int P, int Q>
-__device__ __forceinline__ void emf_edge_partials(const Geo& g, const AdjCell& p,
-                                                  const StageIn& in, const Sweeps& sw,
-                                                  const AdjArrays& A)
+__device__ __forceinline__ void emf_edge_partials(const AdjOffs& of, const StageIn& in,
+                                                  const Sweeps& sw, const AdjArrays& A)
 {
   constexpr int E = 3 - P - Q;
   constexpr int F = (P == 0 ? 0 : P == 1 ? 1 : 2);
-  const long c = p.c;
-  double o[28];
+  const unsigned c = of.c;
+  double o[12];
 #pragma unroll
-  for (int q = 0; q < 28; q++) o[q] = 0.0;
-  const double le = A.lamE[E][c];
+  for (int q = 0; q < 12; q++) o[q] = 0.0;
+  const double le = at_byte(A.lamE[E], c);
   if (le != 0.0) {
-    const long cP = nbr<P>(g, p, 1), cQ = nbr<Q>(g, p, 1);
-    const long cPQ = cP + (cQ - c);
+    const unsigned cP = c + of.d[P][3], cQ = c + of.d[Q][3];
+    const unsigned cPQ = cP + of.d[Q][3];
     const SweepOut &SP = sw.d[P], &SQ = sw.d[Q];
     const double* vP = in.V[VX1 + P];
     const double* vQ = in.V[VX1 + Q];
     const double* bP = in.b[P];
     const double* bQ = in.b[Q];
-    const bool sxp = SP.SR[c] >= SP.SR[cQ], sxm = SP.SL[c] >= SP.SL[cQ];
-    const bool syp = SQ.SR[c] >= SQ.SR[cP], sym = SQ.SL[c] >= SQ.SL[cP];
+    const bool sxp = at_byte(SP.SR, c) >= at_byte(SP.SR, cQ), sxm = at_byte(SP.SL, c) >= at_byte(SP.SL, cQ);
+    const bool syp = at_byte(SQ.SR, c) >= at_byte(SQ.SR, cP), sym = at_byte(SQ.SL, c) >= at_byte(SQ.SL, cP);
     double x[12];
-    x[0] = sxp ? SP.SR[c] : SP.SR[cQ];
-    x[1] = sxm ? SP.SL[c] : SP.SL[cQ];
-    x[2] = syp ? SQ.SR[c] : SQ.SR[cP];
-    x[3] = sym ? SQ.SL[c] : SQ.SL[cP];
-    const long cQm = nbr<Q>(g, p, -1), cPm = nbr<P>(g, p, -1);
-    const long cQQ = nbr<Q>(g, p, 2), cPP = nbr<P>(g, p, 2);
-    const double dpS = bP[cQ] - bP[c], dmS = bP[c] - bP[cQm];
-    const double dpN = bP[cQQ] - bP[cQ], dmN = bP[cQ] - bP[c];
-    const double dpW = bQ[cP] - bQ[c], dmW = bQ[c] - bQ[cPm];
-    const double dpE = bQ[cPP] - bQ[cP], dmE = bQ[cP] - bQ[c];
-    const double bS = bP[c] + 0.5 * mc_lim2(dpS, dmS);
-    const double bW = bQ[c] + 0.5 * mc_lim2(dpW, dmW);
-    const double bN = bP[cQ] - 0.5 * mc_lim2(dpN, dmN);
-    const double bE = bQ[cP] - 0.5 * mc_lim2(dpE, dmE);
-    const double qSW = vQ[c] + 0.5 * (SP.dv[Q][c] + SQ.dv[Q][c]);
-    const double pSW = vP[c] + 0.5 * (SP.dv[P][c] + SQ.dv[P][c]);
-    const double qSE = vQ[cP] - 0.5 * (SP.dv[Q][cP] - SQ.dv[Q][cP]);
-    const double pSE = vP[cP] - 0.5 * (SP.dv[P][cP] - SQ.dv[P][cP]);
-    const double qNE = vQ[cPQ] - 0.5 * (SP.dv[Q][cPQ] + SQ.dv[Q][cPQ]);
-    const double pNE = vP[cPQ] - 0.5 * (SP.dv[P][cPQ] + SQ.dv[P][cPQ]);
-    const double qNW = vQ[cQ] + 0.5 * (SP.dv[Q][cQ] - SQ.dv[Q][cQ]);
-    const double pNW = vP[cQ] + 0.5 * (SP.dv[P][cQ] - SQ.dv[P][cQ]);
+    x[0] = sxp ? at_byte(SP.SR, c) : at_byte(SP.SR, cQ);
+    x[1] = sxm ? at_byte(SP.SL, c) : at_byte(SP.SL, cQ);
+    x[2] = syp ? at_byte(SQ.SR, c) : at_byte(SQ.SR, cP);
+    x[3] = sym ? at_byte(SQ.SL, c) : at_byte(SQ.SL, cP);
+    const unsigned cQm = c + of.d[Q][1], cPm = c + of.d[P][1];
+    const unsigned cQQ = c + of.d[Q][4], cPP = c + of.d[P][4];
+    const double dpS = at_byte(bP, cQ) - at_byte(bP, c), dmS = at_byte(bP, c) - at_byte(bP, cQm);
+    const double dpN = at_byte(bP, cQQ) - at_byte(bP, cQ), dmN = at_byte(bP, cQ) - at_byte(bP, c);
+    const double dpW = at_byte(bQ, cP) - at_byte(bQ, c), dmW = at_byte(bQ, c) - at_byte(bQ, cPm);
+    const double dpE = at_byte(bQ, cPP) - at_byte(bQ, cP), dmE = at_byte(bQ, cP) - at_byte(bQ, c);
+    const double bS = at_byte(bP, c) + 0.5 * mc_lim2(dpS, dmS);
+    const double bW = at_byte(bQ, c) + 0.5 * mc_lim2(dpW, dmW);
+    const double bN = at_byte(bP, cQ) - 0.5 * mc_lim2(dpN, dmN);
+    const double bE = at_byte(bQ, cP) - 0.5 * mc_lim2(dpE, dmE);
+    const double qSW = at_byte(vQ, c) + 0.5 * (at_byte(SP.dv[Q], c) + at_byte(SQ.dv[Q], c));
+    const double pSW = at_byte(vP, c) + 0.5 * (at_byte(SP.dv[P], c) + at_byte(SQ.dv[P], c));
+    const double qSE = at_byte(vQ, cP) - 0.5 * (at_byte(SP.dv[Q], cP) - at_byte(SQ.dv[Q], cP));
+    const double pSE = at_byte(vP, cP) - 0.5 * (at_byte(SP.dv[P], cP) - at_byte(SQ.dv[P], cP));
+    const double qNE = at_byte(vQ, cPQ) - 0.5 * (at_byte(SP.dv[Q], cPQ) + at_byte(SQ.dv[Q], cPQ));
+    const double pNE = at_byte(vP, cPQ) - 0.5 * (at_byte(SP.dv[P], cPQ) + at_byte(SQ.dv[P], cPQ));
+    const double qNW = at_byte(vQ, cQ) + 0.5 * (at_byte(SP.dv[Q], cQ) - at_byte(SQ.dv[Q], cQ));
+    const double pNW = at_byte(vP, cQ) + 0.5 * (at_byte(SP.dv[P], cQ) - at_byte(SQ.dv[P], cQ));
     x[4] = qSW * bS - pSW * bW;
     x[5] = qSE * bS - pSE * bE;
     x[6] = qNE * bN - pNE * bE;
@@ -220,47 +248,15 @@ __device__ __forceinline__ void emf_edge_partials(const Geo& g, const AdjCell& p
     x[11] = bE;
     double ax[12] = {0};
     uct_hll_vjp(x, le, ax);
-    o[0] = ax[0];
-    o[2] = ax[1];
-    o[4] = ax[2];
-    o[6] = ax[3];
-    o[8] = ax[4] * bS;
-    o[9] = -ax[4] * bW;
-    o[10] = ax[5] * bS;
-    o[11] = -ax[5] * bE;
-    o[12] = ax[6] * bN;
-    o[13] = -ax[6] * bE;
-    o[14] = ax[7] * bN;
-    o[15] = -ax[7] * bW;
-    const double abS = ax[8] + ax[4] * qSW + ax[5] * qSE;
-    const double abN = ax[9] + ax[6] * qNE + ax[7] * qNW;
-    const double abW = ax[10] - ax[4] * pSW - ax[7] * pNW;
-    const double abE = ax[11] - ax[5] * pSE - ax[6] * pNE;
-    double adp, adm;
-    adp = adm = 0.0;
-    mc_lim2_vjp(dpS, dmS, 0.5 * abS, adp, adm);
-    o[16] = abS - adp + adm;
-    o[17] = adp;
-    o[18] = -adm;
-    adp = adm = 0.0;
-    mc_lim2_vjp(dpN, dmN, -0.5 * abN, adp, adm);
-    o[19] = abN - adp + adm;
-    o[20] = adp;
-    o[21] = -adm;
-    adp = adm = 0.0;
-    mc_lim2_vjp(dpW, dmW, 0.5 * abW, adp, adm);
-    o[22] = abW - adp + adm;
-    o[23] = adp;
-    o[24] = -adm;
-    adp = adm = 0.0;
-    mc_lim2_vjp(dpE, dmE, -0.5 * abE, adp, adm);
-    o[25] = abE - adp + adm;
-    o[26] = adp;
-    o[27] = -adm;
+#pragma unroll
+    for (int q = 0; q < 8; q++) o[q] = ax[q];
+    o[8] = ax[8] + ax[4] * qSW + ax[5] * qSE;
+    o[9] = ax[9] + ax[6] * qNE + ax[7] * qNW;
+    o[10] = ax[10] - ax[4] * pSW - ax[7] * pNW;
+    o[11] = ax[11] - ax[5] * pSE - ax[6] * pNE;
   }
 #pragma unroll
-  for (int q = 0; q < 28; q++)
-    if (q >= 8 || !(q & 1)) A.ep[F][q][c] = o[q];
+  for (int q = 0; q < 12; q++) at_byte(A.ep[F][q], c) = o[q];
 }
 
 __global__ void __launch_bounds__(256)
@@ -268,77 +264,108 @@ k_adj_emf_partials(Geo g, StageIn in, Sweeps sw, AdjArrays A)
 {
   AdjCell p;
   if (!adj_cell(g, p)) return;
-  emf_edge_partials<0, 1>(g, p, in, sw, A);   // Ez
-  emf_edge_partials<1, 2>(g, p, in, sw, A);   // Ex
-  emf_edge_partials<2, 0>(g, p, in, sw, A);   // Ey
+  const AdjOffs of = adj_offs(g, p);
+  emf_edge_partials<0, 1>(of, in, sw, A);   // Ez
+  emf_edge_partials<1, 2>(of, in, sw, A);   // Ex
+  emf_edge_partials<2, 0>(of, in, sw, A);   // Ey
 }
 
-// periodic neighbour of p at offsets (di, dj, dk), each in [-2, 2]
-__device__ __forceinline__ long nbr3(const Geo& g, const AdjCell& p, int di, int dj, int dk)
+// branch of the MC limiter of the cell between a and b (a, v, b in order): the
+// slope, and its derivatives by the differences b - v and v - a
+struct LimBranch {
+  double s, kp, km;
+};
+
+__device__ __forceinline__ LimBranch lim_branch(double a, double v, double b)
 {
-  int i = p.i + di, j = p.j + dj, k = p.k + dk;
-  i = i < 0 ? i + g.nx : (i >= g.nx ? i - g.nx : i);
-  j = j < 0 ? j + g.ny : (j >= g.ny ? j - g.ny : j);
-  k = k < 0 ? k + g.nz : (k >= g.nz ? k - g.nz : k);
-  return ((long)k * g.ny + j) * g.nx + i;
+  const double dp = b - v, dm = v - a;
+  const double dc = 0.5 * (dp + dm);
+  const bool none = dp * dm < 0.0, small = fabs(dp) < fabs(dm);
+  const double sc = 2.0 * (small ? dp : dm);
+  const bool mid = fabs(dc) < fabs(sc);
+  return {none ? 0.0 : mid ? dc : sc, none ? 0.0 : mid ? 0.5 : small ? 2.0 : 0.0,
+          none ? 0.0 : mid ? 0.5 : small ? 0.0 : 2.0};
 }
 
 template <int P, int Q>
-__device__ __forceinline__ void emf_gather_family(const Geo& g, const AdjCell& p,
-                                                  const AdjArrays& A, const Sweeps& sw,
+__device__ __forceinline__ void emf_gather_family(const AdjOffs& of, const AdjArrays& A,
+                                                  const StageIn& in,
+                                                  const Sweeps& sw,
                                                   double (&sS)[3][2],
                                                   double (&sdv)[3][3], double (&sv)[3],
                                                   double (&sb)[3])
 {
   constexpr int F = (P == 0 ? 0 : P == 1 ? 1 : 2);
-  auto at = [&](int slot, int dp, int dq) {
-    int d[3] = {0, 0, 0};
-    d[P] += dp;
-    d[Q] += dq;
-    return A.ep[F][slot][nbr3(g, p, d[0], d[1], d[2])];
-  };
-  const long c = p.c;
+  auto off = [&](int dp, int dq) { return of.c + of.d[P][dp + 2] + of.d[Q][dq + 2]; };
+  const unsigned c = of.c;
   const double* const* e = A.ep[F];
+  const unsigned cQ = off(0, 1), cQm = off(0, -1), cQmm = off(0, -2), cQQ = off(0, 2);
+  const unsigned cP = off(1, 0), cPm = off(-1, 0), cPmm = off(-2, 0), cPP = off(2, 0);
+  const unsigned cPQm = off(-1, -1);
   // speeds: the max() of edge c picked cell c, that of edge c-Q (c-P)
   // picked its upper cell c (the comparisons of emf_edge_partials)
   {
     const SweepOut &SP = sw.d[P], &SQ = sw.d[Q];
-    int dq[3] = {0, 0, 0}, dp[3] = {0, 0, 0};
-    dq[Q] = 1;
-    dp[P] = 1;
-    const long cQ = nbr3(g, p, dq[0], dq[1], dq[2]), cQm = nbr3(g, p, -dq[0], -dq[1], -dq[2]);
-    const long cP = nbr3(g, p, dp[0], dp[1], dp[2]), cPm = nbr3(g, p, -dp[0], -dp[1], -dp[2]);
-    sS[P][1] += (SP.SR[c] >= SP.SR[cQ] ? e[0][c] : 0.0) + (SP.SR[cQm] >= SP.SR[c] ? 0.0 : e[0][cQm]);
-    sS[P][0] += (SP.SL[c] >= SP.SL[cQ] ? e[2][c] : 0.0) + (SP.SL[cQm] >= SP.SL[c] ? 0.0 : e[2][cQm]);
-    sS[Q][1] += (SQ.SR[c] >= SQ.SR[cP] ? e[4][c] : 0.0) + (SQ.SR[cPm] >= SQ.SR[c] ? 0.0 : e[4][cPm]);
-    sS[Q][0] += (SQ.SL[c] >= SQ.SL[cP] ? e[6][c] : 0.0) + (SQ.SL[cPm] >= SQ.SL[c] ? 0.0 : e[6][cPm]);
+    // (all loaded, then chosen: loads under a condition cost a branch and
+    // 64-bit addresses each, 256 VGPRs instead of 96)
+    auto to_c = [&](const double* sp, const double* part, unsigned lo, unsigned hi) {
+      const double own = at_byte(sp, c), up = at_byte(sp, hi), dn = at_byte(sp, lo);
+      const double pc = at_byte(part, c), pl = at_byte(part, lo);
+      return (own >= up ? pc : 0.0) + (dn >= own ? 0.0 : pl);
+    };
+    sS[P][1] += to_c(SP.SR, e[0], cQm, cQ);
+    sS[P][0] += to_c(SP.SL, e[1], cQm, cQ);
+    sS[Q][1] += to_c(SQ.SR, e[2], cPm, cP);
+    sS[Q][0] += to_c(SQ.SL, e[3], cPm, cP);
   }
+  // limiters along Q of the P faces c-Q, c, c+Q and c-P, along P of the Q
+  // faces c-P, c, c+P and c-Q
+  const double *bP = in.b[P], *bQ = in.b[Q];
+  const double p0 = at_byte(bP, c), pm = at_byte(bP, cQm), pp = at_byte(bP, cQ), pl = at_byte(bP, cPm);
+  const double q0 = at_byte(bQ, c), qm = at_byte(bQ, cPm), qp = at_byte(bQ, cP), ql = at_byte(bQ, cQm);
+  const LimBranch Pm = lim_branch(at_byte(bP, cQmm), pm, p0), P0 = lim_branch(pm, p0, pp), Pp = lim_branch(p0, pp, at_byte(bP, cQQ));
+  const LimBranch Qm = lim_branch(at_byte(bQ, cPmm), qm, q0), Q0 = lim_branch(qm, q0, qp), Qp = lim_branch(q0, qp, at_byte(bQ, cPP));
+  const double sPl = mc_lim2(at_byte(bP, off(-1, 1)) - pl, pl - at_byte(bP, cPQm));
+  const double sQl = mc_lim2(at_byte(bQ, off(1, -1)) - ql, ql - at_byte(bQ, cPQm));
   // corners: c is SW of edge c, SE of c-P, NE of c-P-Q, NW of c-Q
-  const double aSW = e[8][c], pSWv = e[9][c];
-  const double aSE = at(10, -1, 0), pSEv = at(11, -1, 0);
-  const double aNE = at(12, -1, -1), pNEv = at(13, -1, -1);
-  const double aNW = at(14, 0, -1), pNWv = at(15, 0, -1);
+  const double wSW = at_byte(e[4], c), wSE = at_byte(e[5], cPm), wNE = at_byte(e[6], cPQm), wNW = at_byte(e[7], cQm);
+  const double aSW = wSW * (p0 + 0.5 * P0.s), pSWv = -wSW * (q0 + 0.5 * Q0.s);
+  const double aSE = wSE * (pl + 0.5 * sPl), pSEv = -wSE * (q0 - 0.5 * Q0.s);
+  const double aNE = wNE * (pl - 0.5 * sPl), pNEv = -wNE * (ql - 0.5 * sQl);
+  const double aNW = wNW * (p0 - 0.5 * P0.s), pNWv = -wNW * (ql + 0.5 * sQl);
   sv[Q] += aSW + aSE + aNE + aNW;
   sv[P] += pSWv + pSEv + pNEv + pNWv;
   sdv[P][Q] += 0.5 * aSW - 0.5 * aSE - 0.5 * aNE + 0.5 * aNW;
   sdv[Q][Q] += 0.5 * aSW + 0.5 * aSE - 0.5 * aNE - 0.5 * aNW;
   sdv[P][P] += 0.5 * pSWv - 0.5 * pSEv - 0.5 * pNEv + 0.5 * pNWv;
   sdv[Q][P] += 0.5 * pSWv + 0.5 * pSEv - 0.5 * pNEv - 0.5 * pNWv;
-  // faces
-  sb[P] += e[16][c] + at(17, 0, -1) + at(18, 0, 1) + at(19, 0, -1) + at(20, 0, -2) + e[21][c];
-  sb[Q] += e[22][c] + at(23, -1, 0) + at(24, 1, 0) + at(25, -1, 0) + at(26, -2, 0) + e[27][c];
+  // faces: face c is limited as S of edge c and N of c-Q, and is a neighbour
+  // in the limiters of c-Q (S of edge c-Q, N of c-2Q) and c+Q (S of c+Q, N of
+  // c); the same along P for W and E
+  auto faces = [&](const double* lo, const double* hi, unsigned m2, unsigned m1, unsigned p1, const LimBranch& Lm,
+                   const LimBranch& L0, const LimBranch& Lp) {
+    const double l0 = 0.5 * at_byte(lo, c), h0 = -0.5 * at_byte(hi, m1);
+    return (at_byte(lo, c) - L0.kp * l0 + L0.km * l0) + Lm.kp * (0.5 * at_byte(lo, m1)) - Lp.km * (0.5 * at_byte(lo, p1)) +
+           (at_byte(hi, m1) - L0.kp * h0 + L0.km * h0) + Lm.kp * (-0.5 * at_byte(hi, m2)) - Lp.km * (-0.5 * at_byte(hi, c));
+  };
+  sb[P] += faces(e[8], e[9], cQmm, cQm, cQ, Pm, P0, Pp);
+  sb[Q] += faces(e[10], e[11], cPmm, cPm, cP, Qm, Q0, Qp);
 }
 
-__global__ void __launch_bounds__(256) k_adj_emf_gather(Geo g, Sweeps sw, AdjArrays A)
+__global__ void __launch_bounds__(256) k_adj_emf_gather(Geo g, StageIn in, Sweeps sw,
+                                                        AdjArrays A)
 {
   AdjCell p;
   if (!adj_cell(g, p)) return;
+  const AdjOffs of = adj_offs(g, p);
   double sS[3][2] = {{0, 0}, {0, 0}, {0, 0}};
   double sdv[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
   double sv[3] = {0, 0, 0}, sb[3] = {0, 0, 0};
-  emf_gather_family<0, 1>(g, p, A, sw, sS, sdv, sv, sb);
-  emf_gather_family<1, 2>(g, p, A, sw, sS, sdv, sv, sb);
-  emf_gather_family<2, 0>(g, p, A, sw, sS, sdv, sv, sb);
+  emf_gather_family<0, 1>(of, A, in, sw, sS, sdv, sv, sb);
+  asm volatile("" ::: "memory");   // one family's loads at a time
+  emf_gather_family<1, 2>(of, A, in, sw, sS, sdv, sv, sb);
+  asm volatile("" ::: "memory");   // one family's loads at a time
+  emf_gather_family<2, 0>(of, A, in, sw, sS, sdv, sv, sb);
   const long c = p.c;
 #pragma unroll
   for (int d = 0; d < 3; d++) {
@@ -620,7 +647,7 @@ static void adj_stage(const Geo& g, const StageIn& in, const Sweeps& sw, const A
   const dim3 gr = adj_grid(g);
   hipLaunchKernelGGL(k_adj_ct, gr, kAdjBlock, 0, s, g, A, sc);
   hipLaunchKernelGGL(k_adj_emf_partials, gr, kAdjBlock, 0, s, g, in, sw, A);
-  hipLaunchKernelGGL(k_adj_emf_gather, gr, kAdjBlock, 0, s, g, sw, A);
+  hipLaunchKernelGGL(k_adj_emf_gather, gr, kAdjBlock, 0, s, g, in, sw, A);
   // x: whole rows through LDS where they fit a workgroup, else marching
   if (g.nx <= 256) {
     const int nt = (g.nx + 63) / 64 * 64;
@@ -652,7 +679,7 @@ static int adj_alloc(pgpu_domain* d)
 {
   if (d->adj) return PGPU_OK;
   const size_t per = (size_t)d->g.n * sizeof(double);
-  const int narr = 8 + 5 + 5 + 3 + 3 + 3 + 6 + 9 + 3 + 8 + 3 + 84 + 15;
+  const int narr = 8 + 5 + 5 + 3 + 3 + 3 + 6 + 9 + 3 + 8 + 3 + 36 + 15;
   pgpu_adjoint_state* st = new pgpu_adjoint_state;
   st->bytes = per * narr;
   if (hipMalloc(&st->block, st->bytes) != hipSuccess) {
@@ -681,7 +708,7 @@ static int adj_alloc(pgpu_domain* d)
   for (int q = 0; q < 8; q++) A.VN[q] = take();
   for (int a = 0; a < 3; a++) A.bN[a] = take();
   for (int f = 0; f < 3; f++)
-    for (int q = 0; q < 28; q++) A.ep[f][q] = take();
+    for (int q = 0; q < 12; q++) A.ep[f][q] = take();
   for (int dd = 0; dd < 3; dd++)
     for (int q = 0; q < 5; q++) A.sw1[dd][q] = take();
   d->adj = st;
