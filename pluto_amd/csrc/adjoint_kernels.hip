@@ -378,104 +378,163 @@ __global__ void __launch_bounds__(256) k_adj_emf_gather(Geo g, StageIn in, Sweep
   }
 }
 
-// Adjoint of the interface q+1/2 along D (q = cell p): U += -dt/dx
-// (F_{q+1/2} - F_{q-1/2}) and the pressure term, the UCT_HLL face speeds
-// and the velocity slopes of cell q, through HLLD and the MC-limited PLM.
-// part[4 s + k] receives what variable slot s (BN skipped) of the cell at
-// offset k - 1 from q along D gets; the face adjoint of the interface
-// itself is added to lamB when own is set.
-template <int D>
-__device__ __forceinline__ void adj_interface(const Geo& g, const StageIn& in, const AdjArrays& A,
-                                              double dtdx, const AdjCell& p, bool own,
-                                              double part[28])
+// What the adjoint of the interface q+1/2 along D reads besides the primitives
+// of the cells q-1 .. q+2: the adjoints of U of q and q+1, and of cell q the
+// face value, the adjoints of its face speeds and velocity slopes.
+struct Iface {
+  double u0[5], u1[5], b, lS[2], ldv[3];
+};
+
+// Adjoint of the interface q+1/2 along D: U += -dt/dx (F_{q+1/2} -
+// F_{q-1/2}) and the pressure term, the UCT_HLL face speeds and the velocity
+// slopes of cell q, through HLLD and the MC-limited PLM.  cell(k, v) is
+// variable v of the cell q + k, in LDS: it is read again for the limiters, so
+// that its 32 values are not held through the solver.  part[4 s + k]
+// receives what variable slot s (BN skipped) of the cell at offset k - 1 from
+// q along D gets; returns the adjoint of the face value.
+template <int D, typename Cell>
+__device__ __forceinline__ double adj_interface(const Geo& g, const Cell& cell, const Iface& f,
+                                                double dtdx, double part[28])
 {
   constexpr int BN = BX1 + Dir<D>::n;
-  const long c = p.c;
-  const long cm1 = nbr<D>(g, p, -1), cp1 = nbr<D>(g, p, 1), cp2 = nbr<D>(g, p, 2);
-  double vm[NV], v0[NV], vp[NV], vq[NV], vL[NV], vR[NV];
+  double vL[NV], vR[NV];
 #pragma unroll
   for (int q = 0; q < NV; q++) {
-    const double* a = in.V[q];
-    vm[q] = a[cm1];
-    v0[q] = a[c];
-    vp[q] = a[cp1];
-    vq[q] = a[cp2];
-    vL[q] = v0[q] + mc_slope(vm[q], v0[q], vp[q]) * 0.5;
-    vR[q] = vp[q] - mc_slope(v0[q], vp[q], vq[q]) * 0.5;
+    const double v0 = cell(0, q), vp = cell(1, q);
+    vL[q] = v0 + mc_slope(cell(-1, q), v0, vp) * 0.5;
+    vR[q] = vp - mc_slope(v0, vp, cell(2, q)) * 0.5;
   }
-  const double bface = in.b[D][c];
-  vL[BN] = bface;
-  vR[BN] = bface;
+  vL[BN] = f.b;
+  vR[BN] = f.b;
 
   HlldSeed s;
 #pragma unroll
   for (int q = 0; q < NV; q++) s.f[q] = 0.0;
-  s.f[RHO] = dtdx * (A.lamU[0][cp1] - A.lamU[0][c]);
-  s.f[VX1] = dtdx * (A.lamU[1][cp1] - A.lamU[1][c]);
-  s.f[VX2] = dtdx * (A.lamU[2][cp1] - A.lamU[2][c]);
-  s.f[VX3] = dtdx * (A.lamU[3][cp1] - A.lamU[3][c]);
-  s.f[ENG] = dtdx * (A.lamU[4][cp1] - A.lamU[4][c]);
-  s.press = dtdx * (A.lamU[1 + D][cp1] - A.lamU[1 + D][c]);
+  s.f[RHO] = dtdx * (f.u1[0] - f.u0[0]);
+  s.f[VX1] = dtdx * (f.u1[1] - f.u0[1]);
+  s.f[VX2] = dtdx * (f.u1[2] - f.u0[2]);
+  s.f[VX3] = dtdx * (f.u1[3] - f.u0[3]);
+  s.f[ENG] = dtdx * (f.u1[4] - f.u0[4]);
+  s.press = dtdx * (f.u1[1 + D] - f.u0[1 + D]);
   // stored speeds max(0, -SL), max(0, SR): derivative on the active side
   double slmin, slmax, srmin, srmax;
   fast_speeds<D>(vL, g.gamma, slmin, slmax);
   fast_speeds<D>(vR, g.gamma, srmin, srmax);
   const double SL = min_le(slmin, srmin), SR = max_ge(slmax, srmax);
-  s.SL = (0.0 >= -SL) ? 0.0 : -A.lamS[D][0][c];
-  s.SR = (0.0 >= SR) ? 0.0 : A.lamS[D][1][c];
+  s.SL = (0.0 >= -SL) ? 0.0 : -f.lS[0];
+  s.SR = (0.0 >= SR) ? 0.0 : f.lS[1];
 
   double aL[NV] = {0}, aR[NV] = {0};
   hlld_vjp<D>(vL, vR, g.gamma, g.gmm1, s, aL, aR);
-  if (own) A.lamB[D][c] += aL[BN] + aR[BN];
 
+  asm volatile("" ::: "memory");   // the cells are read again from here on
 #pragma unroll
   for (int q = 0; q < NV; q++) {
     if (q == BN) continue;
+    const double vm = cell(-1, q), v0 = cell(0, q), vp = cell(1, q), vq = cell(2, q);
     double a_s0 = 0.5 * aL[q];
-    if (q >= VX1 && q <= VX3) a_s0 += A.lamDV[D][q - VX1][c];
+    if (q >= VX1 && q <= VX3) a_s0 += f.ldv[q - VX1];
     const double a_s1 = -0.5 * aR[q];
     double am = 0.0, a0 = aL[q], ap = aR[q], aq = 0.0;
-    mc_slope_vjp(vm[q], v0[q], vp[q], a_s0, am, a0, ap);
-    mc_slope_vjp(v0[q], vp[q], vq[q], a_s1, a0, ap, aq);
+    mc_slope_vjp(vm, v0, vp, a_s0, am, a0, ap);
+    mc_slope_vjp(v0, vp, vq, a_s1, a0, ap, aq);
     const int sl = 4 * (q < BN ? q : q - 1);
     part[sl + 0] = am;
     part[sl + 1] = a0;
     part[sl + 2] = ap;
     part[sl + 3] = aq;
   }
+  return aL[BN] + aR[BN];
 }
 
-// The x interfaces of one box row (one workgroup, thread i = cell i, nx <=
-// 256): each thread solves the interface i+1/2, the 28 partials go through
-// LDS, and cell i sums what the interfaces i+3/2, i+1/2, i-1/2, i-3/2 sent
-// it into lamV (periodic along the row).
+// The interface adjoints keep about 400 registers a lane, one wave per SIMD, so
+// no other wave hides a load: with each interface's 45 values loaded where they
+// are used they waited for memory 54% of the time.  Both kernels below
+// therefore load what the next interface needs before they solve the present
+// one, take what two interfaces share from registers or LDS, and read the
+// sums that they add to with the same loads.  128^3: x rows 448 -> 260 us a
+// launch, marches 454 -> 255.  (Two waves per SIMD would leave 256 registers a
+// lane: 212 spilled, 741 and 1126 us.)
+
+// The x interfaces of box rows r0 .. r0 + len - 1 of the ny nz rows, one row
+// after another (thread i = cell i, nx <= 256): the row's primitives and U
+// adjoints go through LDS, each thread solves the interface i+1/2, the 28
+// partials go through LDS, and cell i sums what the interfaces i+3/2, i+1/2,
+// i-1/2, i-3/2 sent it into lamV (periodic along the row).
 __global__ void __launch_bounds__(256) k_adj_flux_x_rows(Geo g, StageIn in, AdjArrays A,
-                                                         const DevScalars* sc)
+                                                         const DevScalars* sc, int len)
 {
-  extern __shared__ double sm[];   // [28][blockDim.x]
-  const int nt = blockDim.x, i = threadIdx.x;
-  AdjCell p;
-  p.i = i;
-  p.j = blockIdx.x;
-  p.k = blockIdx.y;
-  p.c = ((long)p.k * g.ny + p.j) * g.nx + i;
-  if (i < g.nx) {
-    double part[28];
-    adj_interface<0>(g, in, A, sc->dt / g.dx[0], p, true, part);
-#pragma unroll
-    for (int m = 0; m < 28; m++) sm[m * nt + i] = part[m];
-  }
-  __syncthreads();
-  if (i >= g.nx) return;
-  const int n1 = i + 1 < g.nx ? i + 1 : i + 1 - g.nx;
+  extern __shared__ double sm[];   // [28][blockDim.x] partials, [13][blockDim.x] cells
+  const int nt = blockDim.x, t = threadIdx.x;
+  double* cell = sm + 28 * nt;
+  const bool act = t < g.nx;
+  const int i = act ? t : g.nx - 1;   // (idle lanes load the last cell)
+  const int r0 = blockIdx.x * len, r1 = min(r0 + len, g.ny * g.nz);
+  const int p1 = i + 1 < g.nx ? i + 1 : i + 1 - g.nx;
+  const int p2 = i + 2 < g.nx ? i + 2 : i + 2 - g.nx;
   const int m1 = i >= 1 ? i - 1 : i - 1 + g.nx;
   const int m2 = i >= 2 ? i - 2 : i - 2 + g.nx;
+  const double dtdx = sc->dt / g.dx[0];
+  struct Row {
+    double v[NV], u[5], b, lS[2], ldv[3], lb, lv[7];
+  };
+  auto load = [&](int r) {
+    const unsigned c = ((unsigned)r * (unsigned)g.nx + (unsigned)i) * 8u;
+    Row w;
 #pragma unroll
-  for (int q = 0; q < NV; q++) {
-    if (q == BX1) continue;
-    const int sl = 4 * (q < BX1 ? q : q - 1);
-    A.lamV[q][p.c] += sm[(sl + 0) * nt + n1] + sm[(sl + 1) * nt + i] +
-                      sm[(sl + 2) * nt + m1] + sm[(sl + 3) * nt + m2];
+    for (int q = 0; q < NV; q++) w.v[q] = at_byte(in.V[q], c);
+#pragma unroll
+    for (int q = 0; q < 5; q++) w.u[q] = at_byte(A.lamU[q], c);
+    w.b = at_byte(in.b[0], c);
+    w.lS[0] = at_byte(A.lamS[0][0], c);
+    w.lS[1] = at_byte(A.lamS[0][1], c);
+#pragma unroll
+    for (int q = 0; q < 3; q++) w.ldv[q] = at_byte(A.lamDV[0][q], c);
+    w.lb = at_byte(A.lamB[0], c);
+#pragma unroll
+    for (int s = 0; s < 7; s++) w.lv[s] = at_byte(A.lamV[s < BX1 ? s : s + 1], c);
+    return w;
+  };
+  Row w = load(r0);
+  for (int r = r0; r < r1; r++) {
+    const unsigned c = ((unsigned)r * (unsigned)g.nx + (unsigned)i) * 8u;
+    if (act) {
+#pragma unroll
+      for (int q = 0; q < NV; q++) cell[q * nt + i] = w.v[q];
+#pragma unroll
+      for (int q = 0; q < 5; q++) cell[(NV + q) * nt + i] = w.u[q];
+    }
+    const Row cur = w;
+    w = load(min(r + 1, r1 - 1));
+    __syncthreads();
+    if (act) {
+      Iface f;
+#pragma unroll
+      for (int q = 0; q < 5; q++) {
+        f.u0[q] = cur.u[q];
+        f.u1[q] = cell[(NV + q) * nt + p1];
+      }
+      f.b = cur.b;
+      f.lS[0] = cur.lS[0];
+      f.lS[1] = cur.lS[1];
+#pragma unroll
+      for (int q = 0; q < 3; q++) f.ldv[q] = cur.ldv[q];
+      double part[28];
+      const double ab = adj_interface<0>(
+          g, [&](int k, int q) { return cell[q * nt + (k < 0 ? m1 : k == 0 ? i : k == 1 ? p1 : p2)]; }, f,
+          dtdx, part);
+      at_byte(A.lamB[0], c) = cur.lb + ab;
+#pragma unroll
+      for (int m = 0; m < 28; m++) sm[m * nt + i] = part[m];
+    }
+    __syncthreads();
+    if (act) {
+#pragma unroll
+      for (int s = 0; s < 7; s++)
+        at_byte(A.lamV[s < BX1 ? s : s + 1], c) =
+            cur.lv[s] + (sm[4 * s * nt + p1] + sm[(4 * s + 1) * nt + i] + sm[(4 * s + 2) * nt + m1] +
+                         sm[(4 * s + 3) * nt + m2]);
+    }
   }
 }
 
@@ -493,6 +552,7 @@ __global__ void __launch_bounds__(256) k_adj_flux_march(Geo g, StageIn in, AdjAr
 {
   constexpr int BN = BX1 + Dir<D>::n;
   __shared__ double ring[28][256];   // [4 * slot + cell (mod 4)][thread]
+  __shared__ double vcell[4 * NV][256];   // the cells q-1 .. q+2: [NV * (cell mod 4) + variable][thread]
   const int t = threadIdx.y * blockDim.x + threadIdx.x;
   const int nD = D == 0 ? g.nx : D == 1 ? g.ny : g.nz;
   const int l0 = blockIdx.x * blockDim.x + threadIdx.x;           // first transverse axis
@@ -504,15 +564,63 @@ __global__ void __launch_bounds__(256) k_adj_flux_march(Geo g, StageIn in, AdjAr
 #pragma unroll
   for (int m = 0; m < 28; m++) ring[m][t] = 0.0;
   const double dtdx = sc->dt / g.dx[D];
+  // byte offset of the line's cell q, periodic
+  const unsigned sD = 8u * (D == 0 ? 1u : D == 1 ? (unsigned)g.nx : (unsigned)g.nx * (unsigned)g.ny);
+  const unsigned base = 8u * (D == 0   ? ((unsigned)l1 * (unsigned)g.ny + (unsigned)l0) * (unsigned)g.nx
+                              : D == 1 ? (unsigned)l1 * (unsigned)g.ny * (unsigned)g.nx + (unsigned)l0
+                                       : (unsigned)l1 * (unsigned)g.nx + (unsigned)l0);
+  auto off = [&](int q) { return base + (unsigned)(q < 0 ? q + nD : q >= nD ? q - nD : q) * sD; };
+  // what an interface does not share with the one before it: cell q+2, the U
+  // adjoint of q+1, what it reads of cell q, and the sums of cell q-1
+  struct Ahead {
+    double vq[NV], u1[5], b, lS[2], ldv[3], lb, lv[7];
+  };
+  auto load = [&](int q) {
+    const unsigned c = off(q), c1 = off(q + 1), c2 = off(q + 2), cm = off(q - 1);
+    Ahead w;
+#pragma unroll
+    for (int v = 0; v < NV; v++) w.vq[v] = at_byte(in.V[v], c2);
+#pragma unroll
+    for (int v = 0; v < 5; v++) w.u1[v] = at_byte(A.lamU[v], c1);
+    w.b = at_byte(in.b[D], c);
+    w.lS[0] = at_byte(A.lamS[D][0], c);
+    w.lS[1] = at_byte(A.lamS[D][1], c);
+#pragma unroll
+    for (int v = 0; v < 3; v++) w.ldv[v] = at_byte(A.lamDV[D][v], c);
+    w.lb = at_byte(A.lamB[D], c);
+#pragma unroll
+    for (int s = 0; s < 7; s++) w.lv[s] = at_byte(A.lamV[s < BN ? s : s + 1], cm);
+    return w;
+  };
+  Iface f;
+  Ahead w = load(q0 - 2);
+  {
+    const unsigned cm = off(q0 - 3), c = off(q0 - 2), c1 = off(q0 - 1);
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      vcell[NV * ((q0 - 3) & 3) + v][t] = at_byte(in.V[v], cm);
+      vcell[NV * ((q0 - 2) & 3) + v][t] = at_byte(in.V[v], c);
+      vcell[NV * ((q0 - 1) & 3) + v][t] = at_byte(in.V[v], c1);
+    }
+#pragma unroll
+    for (int v = 0; v < 5; v++) f.u0[v] = at_byte(A.lamU[v], c);
+  }
   for (int q = q0 - 2; q <= q1; q++) {
-    const int qw = q < 0 ? q + nD : q >= nD ? q - nD : q;
-    AdjCell p;
-    p.i = D == 0 ? qw : l0;
-    p.j = D == 1 ? qw : D == 0 ? l0 : l1;
-    p.k = D == 2 ? qw : l1;
-    p.c = ((long)p.k * g.ny + p.j) * g.nx + p.i;
+    const Ahead cur = w;
+    w = load(min(q + 1, q1));
+#pragma unroll
+    for (int v = 0; v < NV; v++) vcell[NV * ((q + 2) & 3) + v][t] = cur.vq[v];
+#pragma unroll
+    for (int v = 0; v < 5; v++) f.u1[v] = cur.u1[v];
+    f.b = cur.b;
+    f.lS[0] = cur.lS[0];
+    f.lS[1] = cur.lS[1];
+#pragma unroll
+    for (int v = 0; v < 3; v++) f.ldv[v] = cur.ldv[v];
     double part[28];
-    adj_interface<D>(g, in, A, dtdx, p, q >= q0 && q < q1, part);
+    const double ab = adj_interface<D>(
+        g, [&](int k, int v) { return vcell[NV * ((q + k) & 3) + v][t]; }, f, dtdx, part);
+    if (q >= q0 && q < q1) at_byte(A.lamB[D], off(q)) = cur.lb + ab;
     // targets q-1 .. q+2 (k = 0..3) sit in ring slots (q - 1 + k) mod 4
 #pragma unroll
     for (int s = 0; s < 7; s++)
@@ -521,17 +629,14 @@ __global__ void __launch_bounds__(256) k_adj_flux_march(Geo g, StageIn in, AdjAr
     // cell q-1 is complete: its last interface was q+1/2
     const int done = (q - 1) & 3;
     if (q - 1 >= q0) {
-      const int cw = q - 1 < 0 ? q - 1 + nD : q - 1;
-      const long cc = p.c + (long)(cw - qw) * (D == 0 ? 1L : D == 1 ? (long)g.nx : (long)g.nx * g.ny);
+      const unsigned cc = off(q - 1);
 #pragma unroll
-      for (int v = 0; v < NV; v++) {
-        if (v == BN) continue;
-        const int s = v < BN ? v : v - 1;
-        A.lamV[v][cc] += ring[4 * s + done][t];
-      }
+      for (int s = 0; s < 7; s++) at_byte(A.lamV[s < BN ? s : s + 1], cc) = cur.lv[s] + ring[4 * s + done][t];
     }
 #pragma unroll
     for (int s = 0; s < 7; s++) ring[4 * s + done][t] = 0.0;
+#pragma unroll
+    for (int v = 0; v < 5; v++) f.u0[v] = f.u1[v];
   }
 }
 
@@ -640,6 +745,17 @@ static int adj_march_len(const Geo& g, int D)
   return len;
 }
 
+// Rows a workgroup of the x interfaces takes one after another (only the first
+// one's loads are waited for): 16, fewer where that would leave less than two
+// workgroups for each place (four waves a CU)
+static int adj_rows_len(int rows, int nt)
+{
+  const int places = 256 * (256 / nt);
+  int len = 16;
+  while (len > 1 && (rows + len - 1) / len < 2 * places) len /= 2;
+  return len;
+}
+
 // One stage in reverse: CT transpose, EMF adjoint, flux adjoints.
 static void adj_stage(const Geo& g, const StageIn& in, const Sweeps& sw, const AdjArrays& A,
                       const DevScalars* sc, hipStream_t s)
@@ -651,8 +767,9 @@ static void adj_stage(const Geo& g, const StageIn& in, const Sweeps& sw, const A
   // x: whole rows through LDS where they fit a workgroup, else marching
   if (g.nx <= 256) {
     const int nt = (g.nx + 63) / 64 * 64;
-    hipLaunchKernelGGL(k_adj_flux_x_rows, dim3(g.ny, g.nz), dim3(nt), 28 * nt * sizeof(double), s,
-                       g, in, A, sc);
+    const int rows = g.ny * g.nz, len = adj_rows_len(rows, nt);
+    hipLaunchKernelGGL(k_adj_flux_x_rows, dim3((rows + len - 1) / len), dim3(nt),
+                       41 * nt * sizeof(double), s, g, in, A, sc, len);
   } else {
     const int len = adj_march_len(g, 0);
     hipLaunchKernelGGL(k_adj_flux_march<0>, dim3((g.ny + 63) / 64, (g.nz + 3) / 4, (g.nx + len - 1) / len),

@@ -292,6 +292,35 @@ def test_adjoint_of_tiled_box_equals_tiled_adjoint(native):
         assert err <= 1e-12
 
 
+# x rows of one, two and four waves, 1, 8 and 16 of them a workgroup with the
+# last group cut, the x march, y and z segments with remainders; the 5^3 tile
+# itself takes one row a workgroup and one segment
+@pytest.mark.parametrize("reps", [(3, 7, 12), (41, 40, 12), (27, 20, 25), (13, 14, 51), (5, 3, 52)])
+def test_adjoint_of_tiled_boxes(native, reps):
+    from pluto_amd import problems as P
+    from pluto_amd.adjoint import Stepper, cfl_dt
+    torch = _torch()
+    _say("case: adjoint of 5^3 tiled %s, 2 steps" % (reps,))
+    st = P.random_mhd_3d(5, seed=47, v_rms=0.3, b_rms=0.4)
+    dt = cfl_dt(st, 0.3)
+    rng = np.random.default_rng(53)
+    wp, wf = rng.standard_normal((8,) + st.shape), rng.standard_normal((3,) + st.shape)
+
+    def tile(a):
+        return np.ascontiguousarray(np.tile(a, (1,) + reps))
+
+    small = Stepper(st.shape, st.spacing(), dt)
+    gp, gf = _grad_linear(small, *_state_tensors(st), 2, wp, wf)
+    small.close()
+    big = Stepper(tuple(s * r for s, r in zip(st.shape, reps)), st.spacing(), dt)
+    big_state = [torch.tensor(tile(a), dtype=torch.float64, device="cuda").contiguous()
+                 for a in (st.prim, np.stack([st.bx, st.by, st.bz]))]
+    Gp, Gf = _grad_linear(big, *big_state, 2, tile(wp), tile(wf))
+    big.close()
+    for a, b in ((Gp, tile(gp)), (Gf, tile(gf))):   # up to the order of the sums
+        assert np.abs(a - b).max() <= 1e-12 * np.abs(b).max()
+
+
 def test_one_step_gradient_vs_oracle_differences(native, oracle_lib):
     """The FD reference computed with the oracle's forward step.
 
