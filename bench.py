@@ -49,10 +49,10 @@ METRIC = "Mzone-updates/s 256³ HLLD+CT: plain FP64 vs FP32-flux; adjoint/forwar
 # Stage-1 and stage-2 launches alternate, so each entry is their mean.
 KERNEL_BYTES = {
     # fused pipeline (default)
-    "flux_xy": 0.5 * (208.0 + 240.0),  # V 8, bx by 2, (U 5); U 5, S 4, dv 6, (C_dt 1)
-    "flux_z": 0.5 * (200.0 + 192.0),   # V 8, bz 1, U 5, (C_dt 1); U 5, S 2, dv 3
-    "emf": 192.0,                      # S 6, dv 9, v 3, faces 3; edges 3
-    "ct": 0.5 * (216.0 + 264.0),       # edges 3, faces 3, U 5, (b0 3, V 8); faces 3, V 8, (U 5)
+    "flux_xy": 0.5 * (160.0 + 192.0),  # V 8, bx by 2, (U 5); U 5, S 4, (C_dt 1)
+    "flux_z": 0.5 * (176.0 + 168.0),   # V 8, bz 1, U 5, (C_dt 1); U 5, S 2
+    "emf": 120.0,                      # S 6, v 3, faces 3; edges 3
+    "ct": 0.5 * (176.0 + 264.0),       # edges 3, faces 3, U 5, (b0 3, V 8); faces 3, V 8, (U 5)
     # modular pipeline
     "sweep_x": 168.0, "sweep_y": 168.0, "sweep_z": 168.0,
     "update": 0.5 * (272.0 + 248.0),

@@ -198,17 +198,16 @@ int  pgpu_set_emf_tiling (int bx, int by, int kz);
 int  pgpu_get_emf_tiling (int *bx, int *by, int *kz);
 /* UCT_HLL EMF kernel of FP64 3D boxes (process-wide; results identical):
    0 the register-rolling z-march (tiled by pgpu_set_emf_tiling); the
-   LDS-staged z-march (boxes with nx even) with column tiles of 1: 64 x 4,
-   2: 32 x 4, 3: 32 x 8 (the default); kz planes per workgroup (0: 16). */
+   LDS-staged z-march with column tiles of 1: 64 x 4, 2: 32 x 4, 3: 32 x 8
+   (the default; also what 2D boxes take); kz planes per workgroup (0: 16). */
 int  pgpu_set_emf_kernel (int kind, int kz);
 /* x/y flux kernel of the fused step (process-wide; FP64 results identical,
    FP32-flux results equal to FP32 rounding, 5e-7 relative):
-   0 overlapping z-plane tiles; 1 (the default) one workgroup per box row
-   marching up y segments of seg rows (0: 32, fewer on boxes too small to
-   fill the GPU with 32-row segments), each cell reconstructed
-   once per direction, on boxes with nx even (a multiple of 4 for the
-   FP32-flux path) and <= 256, ny >= 4 and fields under 4 GiB; the tiles
-   elsewhere. */
+   0 overlapping z-plane tiles; 1 (the default) workgroups of whole box rows,
+   or of windows of them (rows wider than 256 cells among others), marching
+   up y segments of seg rows (0: by size, 32 at most), each cell
+   reconstructed once per direction, on boxes with fields under 4 GiB; with
+   seg 0 small FP64 boxes still take the tiles where those are faster. */
 int  pgpu_set_flux_kernel (int kind, int seg);
 
 /* Host <-> device state copies (synchronous).  prim is [8][nz][ny][nx];

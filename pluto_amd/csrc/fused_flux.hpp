@@ -8,10 +8,11 @@
 // AdvanceStep).  Same arithmetic as the modular kernels in stage_kernels.hip
 // (and thus as the reference), organised to move fewer bytes:
 //
-//   k_flux_xy_rows    (the default x/y kernel) one workgroup per box row,
-//                     marching up a y segment: each cell reconstructed once
-//                     per direction, x neighbours through LDS, y carried in
-//                     registers (see the kernel).
+//   k_flux_xy_rows    (the default x/y kernel) a workgroup holds whole box
+//                     rows, or a window of the rows of all planes one after
+//                     another, and marches up a y segment: each cell
+//                     reconstructed once per direction, x neighbours through
+//                     LDS, y carried in registers (see the kernel).
 //   k_flux_xy<STAGE>  one z-plane tile per workgroup.  The primitive state of
 //                     the tile plus its stencil halo is staged in LDS once;
 //                     each thread solves one x and one y interface (PLM +

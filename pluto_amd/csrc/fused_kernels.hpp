@@ -77,7 +77,8 @@ int flux_xy_seg();
 // 176 (one row: 180, and 299 against 206 at 32 rows), 64^3 36 (one row a
 // workgroup: 47), 16 x 256^2 91 (windows of one row: 196), 133^3 windows
 // 8 rows 278 (32: 304), 261 x 256^2 16 rows 1345 (8: 1434), 384 x 288 x 320
-// 2790 (tiles: 3792).
+// 2790 (tiles: 3792).  (Both kernels wrote the velocity slopes then; without
+// them every figure is about 7% less, 256^3 1180 and 384 x 288 x 320 2570.)
 struct RowLaunch {
   int nt = 0, wgs = 0, rows = 0, seg = 0;
 };

@@ -207,7 +207,7 @@ def set_emf_tiling(bx: int = 0, by: int = 0, kz: int = 0) -> None:
 
 
 def set_emf_kernel(kind: int = 3, kz: int = 0) -> None:
-    """UCT_HLL EMF kernel of FP64 3D boxes (process-wide): 0 register z-march,
+    """UCT_HLL EMF kernel of the fused step (process-wide): 0 register z-march,
     LDS-staged with tiles 1: 64 x 4, 2: 32 x 4, 3: 32 x 8 (default); kz
     planes per workgroup (0: 16).  Results do not depend on it."""
     check(lib().pgpu_set_emf_kernel(int(kind), int(kz)))
@@ -215,8 +215,9 @@ def set_emf_kernel(kind: int = 3, kz: int = 0) -> None:
 
 def set_flux_kernel(kind: int = 1, seg: int = 0) -> None:
     """x/y flux kernel of the fused step (process-wide): 0 overlapping
-    z-plane tiles, 1 row workgroups marching up y segments of seg rows
-    (0: by size; the default).  FP64 results do not depend on it; the
+    z-plane tiles, 1 workgroups of rows or windows of rows marching up y
+    segments of seg rows (0: by size, and the tiles on small FP64 boxes where
+    those are faster; the default).  FP64 results do not depend on it; the
     FP32-flux path's differ in the last FP32 bits (contraction)."""
     check(lib().pgpu_set_flux_kernel(int(kind), int(seg)))
 
