@@ -111,12 +111,20 @@ k_emf_zs(Geo g, StageIn in, Sweeps sw, EdgeOut e, int kz)
   const int tx = threadIdx.x, ty = threadIdx.y, tid = tx + TX * ty;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int i0 = blockIdx.x * TX, j0 = blockIdx.y * TY;
+  // shortened segments (boxes that 16 planes a workgroup would not fill): tiles
+  // numbered so that each XCD runs one contiguous range of them and finds the
+  // halos in its L2.  us a launch, plain and so: 64^3 26.3 and 23.2, 96^3 71.3
+  // and 62, 128^3 117 and 108, 160^3 211 and 196, 192^3 322 and 307.  Not where
+  // all workgroups run at once (32^3: the divisions cost more), nor with whole
+  // segments (256^3 683 and 703, 384 x 288 x 320 1511 and 1530)
+  const unsigned wgs = gridDim.x * gridDim.y * gridDim.z;
+  const dim3 tb = D3 && kz < 16 && wgs > 512u ? xcd_tile() : dim3(blockIdx.x, blockIdx.y, blockIdx.z);
+  const int i0 = tb.x * TX, j0 = tb.y * TY;
   const int i = i0 + tx, j = j0 + ty;
   const bool active = i < g.nx && j < g.ny;
   const EmfFields f = emf_fields(in, sw);
   const unsigned nxy = (unsigned)g.nx * (unsigned)g.ny;
-  const ZSeg zs = zseg(g, blockIdx.z, kz);   // (a patch of a stack: z periodic within it)
+  const ZSeg zs = zseg(g, tb.z, kz);   // (a patch of a stack: z periodic within it)
 
   // in-plane byte offsets of this lane in the chunks its wave copies
   // (chunk c of every footprint goes to wave c % NW)

@@ -284,8 +284,9 @@ __device__ __forceinline__ int wrap2(int q, int o, int n)
 // XCD at about the same time, and the halo comes from its L2 instead of HBM.
 // A bijection for any grid size, so it changes which workgroup computes a
 // tile, never what is computed.  It pays in the overlapping FP64 x/y flux
-// tile (about 2.5% at 256^3); in the z-marching EMF and CT kernels and the
-// FP32 tile it measured slightly slower, so they keep the plain numbering.
+// tile (about 2.5% at 256^3), the row kernel and the LDS EMF of smaller boxes;
+// in the z-marching CT kernel and the FP32 tile it measured slightly slower, so
+// they keep the plain numbering.
 __device__ __forceinline__ dim3 xcd_tile()
 {
   const unsigned gx = gridDim.x, gy = gridDim.y;
