@@ -50,20 +50,22 @@ struct FillSide {
   int nop, dir, end_side, kind;   // kind: 0 outflow, 1 periodic, 2 reflective
 };
 
-// one side, or both sides of an axis (blockIdx.z): neither reads a cell that
-// the other writes (a box has as many interior cells as ghost zones)
+// one side, or both sides of an axis (blockIdx.z): neither reads an element
+// that the other writes.  A box has as many interior cells as ghost zones, so
+// the sources are interior, but for the periodic normal face: there the
+// beginning's side copies face end to face beg-1, and the end's side, whose
+// face box starts one face below its ghost cells, would copy beg-1 to end.  One
+// after the other that second copy changes nothing; in one launch the two
+// race, so the end's box starts at end+1 there (fill_sides).
 struct FillSides {
   FillSide side[2];
 };
 
-__global__ void __launch_bounds__(256) k_bound_fill(GhostBox b, FillSides fs)
+// line t (a transverse point) of copy o of side f
+__device__ __host__ inline void fill_line(const GhostBox& b, const FillSide& f, const FillOp& o, long t)
 {
-  const FillSide& f = fs.side[blockIdx.z];
-  if ((int)blockIdx.y >= f.nop) return;
-  const FillOp& o = f.op[blockIdx.y];
   const int d = f.dir, ta = d == 0 ? 1 : 0, tb = d == 2 ? 1 : 2;
   const int na = o.hi[ta] - o.lo[ta] + 1, nb = o.hi[tb] - o.lo[tb] + 1;
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long)na * nb) return;
   int p[3];
   p[ta] = o.lo[ta] + (int)(t % na);
@@ -79,6 +81,13 @@ __global__ void __launch_bounds__(256) k_bound_fill(GhostBox b, FillSides fs)
     const double v = o.p[gidx(b, o.ext, q[0], q[1], q[2])];
     o.p[gidx(b, o.ext, p[0], p[1], p[2])] = f.kind == 2 ? o.sgn * v : v;
   }
+}
+
+__global__ void __launch_bounds__(256) k_bound_fill(GhostBox b, FillSides fs)
+{
+  const FillSide& f = fs.side[blockIdx.z];
+  if ((int)blockIdx.y >= f.nop) return;
+  fill_line(b, f, f.op[blockIdx.y], (long)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 struct DivbSide {
@@ -187,9 +196,10 @@ static int launch_divb(const GhostBox& b, const DivbSides& g, int sides, hipStre
   return (int)hipGetLastError();
 }
 
-// the copies of one side; the transverse points of its largest box into most
+// the copies of one side; the transverse points of its largest box into most.
+// both: the end's side in a launch with its axis' periodic beginning
 static int fill_side(const GhostBox& b, int side, int type, double* const* vc, double* const* vs,
-                     FillSide& f, long& most)
+                     bool both, FillSide& f, long& most)
 {
   if (side < 0 || side > 5) return (int)hipErrorInvalidValue;
   const int d = side / 2, end_side = side & 1;
@@ -231,9 +241,26 @@ static int fill_side(const GhostBox& b, int side, int type, double* const* vc, d
   for (int a = 0; a < 3; a++) {
     if (a == d && f.kind != 1) continue;
     int l[3] = {lo[0], lo[1], lo[2]}, h[3] = {hi[0], hi[1], hi[2]};
-    if (l[a] < h[a]) l[a] -= 1;
-    else h[a] -= 1;
+    if (a == d && both) {
+      // (face end is the beginning's source)
+    } else if (l[a] < h[a]) {
+      l[a] -= 1;
+    } else {
+      h[a] -= 1;
+    }
     add(vs[a], a, l, h, sgn[kBX1 + a]);
+  }
+  return 0;
+}
+
+// the copies of side `first`, or of it and the next (sides 2: an axis)
+static int fill_sides(const GhostBox& b, int first, const int* type, int sides, double* const* vc,
+                      double* const* vs, FillSides& f, long& most)
+{
+  for (int q = 0; q < sides; q++) {
+    const bool both = q == 1 && type[0] == BOUND_PERIODIC && type[1] == BOUND_PERIODIC;
+    const int rc = fill_side(b, first + q, type[q], vc, vs, both, f.side[q], most);
+    if (rc) return rc;
   }
   return 0;
 }
@@ -245,10 +272,10 @@ static int launch_sides(const GhostBox& b, int first, const int* type, int sides
   FillSides f{};
   DivbSides g{};
   long most = 0;
+  const int rc = fill_sides(b, first, type, sides, vc, vs, f, most);
+  if (rc) return rc;
   int nop = 0, nd = 0;
   for (int q = 0; q < sides; q++) {
-    const int rc = fill_side(b, first + q, type[q], vc, vs, f.side[q], most);
-    if (rc) return rc;
     nop = f.side[q].nop > nop ? f.side[q].nop : nop;
     if (f.side[q].kind == 1) continue;
     if (!area && !area_c) return (int)hipErrorInvalidValue;

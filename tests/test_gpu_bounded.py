@@ -408,3 +408,75 @@ def test_bounded_userdef_hook_vs_pluto(native, bounds):
     with pytest.raises(native.PGPUError, match="USERDEF"):
         dom.run(1)
     dom.close()
+
+
+def _lower(faces):
+    """The last face planes: what lies below the first cells of a periodic box."""
+    bx, by, bz = faces
+    return [bx[:, :, -1].copy(), by[:, -1, :].copy(), bz[-1].copy()]
+
+
+def _centres_with(st, low):
+    """The first cells' centred field as set_state(low=...) forms it."""
+    st.prim[4][:, :, 0] = 0.5 * (st.bx[:, :, 0] + low[0])
+    st.prim[5][:, 0, :] = 0.5 * (st.by[:, 0, :] + low[1])
+    st.prim[6][0] = 0.5 * (st.bz[0] + low[2])
+
+
+def _bounded_vs_oracle(native, st, low, bounds, nghost, what):
+    from oracle import oracle as O
+    dom = native.Domain(st.shape, 3, st.spacing(), bounds=bounds, nghost=nghost)
+    dom.set_state(st, low=low)
+    dom.set_dt(1e-3, 0.3, 1.1)
+    dom.run(3)
+    out = dom.get_state(st)
+    lows = dom.low_faces()
+    dom.close()
+    ref = st.copy()
+    _centres_with(ref, low)
+    O.run(ref, 3, 1e-3, cfl=0.3)
+    assert_states_equal(out, ref, what)
+    return lows, _lower((ref.bx, ref.by, ref.bz))
+
+
+# the ghost fill of periodic axes, the faces below the first cells differing
+# from the last faces (which the fill replaces them by): extents equal to the
+# ghost zones, odd and larger ones
+@pytest.mark.parametrize("shape,nghost", [((3, 3, 3), 3), ((5, 7, 9), 2), ((12, 5, 17), 4), ((33, 20, 70), 2)])
+def test_periodic_sides_with_other_lower_faces(native, shape, nghost):
+    _say("case: bounded all-periodic %s, %d ghost zones, lower faces of their own" % (shape, nghost))
+    st = _box(shape, seed=61)
+    rng = np.random.default_rng(67)
+    low = [a + 0.05 * rng.standard_normal(a.shape) for a in _lower((st.bx, st.by, st.bz))]
+    lows, ref = _bounded_vs_oracle(native, st, low, ("periodic",) * 6, nghost, "all periodic %s" % (shape,))
+    for a, b in zip(lows, ref):
+        assert np.array_equal(a, b)
+
+
+# periodic axes before outflow ones (X1 is filled first, X3 last: an outflow
+# fill reads the faces below the first cells of the periodic axes after it as
+# they were): a state that varies along one periodic axis only, so that an
+# outflow ghost zone holds what a periodic one does (exactly: face areas are
+# powers of two and the other axes' differences vanish)
+@pytest.mark.parametrize("axis,periodic", [(0, 1), (0, 2), (1, 2)])
+@pytest.mark.parametrize("extents,nghost", [((9, 4, 3), 2), ((3, 3, 3), 3), ((70, 5, 8), 2)])
+def test_periodic_axes_before_outflow(native, axis, periodic, extents, nghost):
+    from pluto_amd import problems as P
+    n = [extents[(a - axis) % 3] for a in range(3)]   # x, y, z
+    shape = (n[2], n[1], n[0])
+    _say("case: bounded %s varying along axis %d, the first %d axes periodic" % (shape, axis, periodic))
+    rng = np.random.default_rng(71)
+    line = [1] * 3
+    line[2 - axis] = n[axis]
+
+    def wave(lo, amp):
+        return np.broadcast_to((lo + amp * rng.standard_normal(n[axis])).reshape(line), shape).copy()
+
+    b = [wave(0.3, 0.2) for _ in range(3)]
+    b[axis][:] = 0.75
+    v = np.stack([wave(0.0, 0.3) for _ in range(3)])
+    st = P.assemble(wave(1.0, 0.1), v, wave(1.0, 0.1), *b, 3, tuple(0.25 * x for x in n))
+    low = _lower(b)
+    low[axis] += 0.0625
+    bounds = ["periodic" if a < periodic else "outflow" for a in (0, 0, 1, 1, 2, 2)]
+    _bounded_vs_oracle(native, st, low, bounds, nghost, "axis %d of %s" % (axis, shape))
