@@ -781,9 +781,11 @@ static int enqueue_step_fused(pgpu_domain* d)
   ends.cfl_max_var = d->cfl_max_var;
   if (sig) rc = launch_sig_sweep(g, in1, d->sig, d->stream);
   if (!rc) rc = flux(1, in1, U, fd);
+  if (!rc) rc = launch_emf(g, in1, d->sw, d->e, d->stream, kt, fp32);
+  // (after the EMF: the slopes take the arrays that hold the face mass flux of
+  // the other EMF averages, which may be chosen while the signature is on)
   if (!rc && sig) rc = launch_vel_slopes(g, in1, d->sw, d->stream);
   if (!rc && sig) rc = launch_sig_emf(g, in1, d->sw, d->sig, d->stream);
-  if (!rc) rc = launch_emf(g, in1, d->sw, d->e, d->stream, kt, fp32);
   // the FP32-flux path stores V1 (read only by stage 2's FP32 flux and EMF
   // kernels) as float
   if (!rc) rc = launch_ct_c2p(g, 1, d->e, fA, fA, oB, U, vn, V1, d->flag, d->sc, d->stream, kt, fp32, ends);
@@ -793,9 +795,9 @@ static int enqueue_step_fused(pgpu_domain* d)
   if (rc) return rc;
   if (sig) rc = launch_sig_sweep(g, in2, d->sig, d->stream);
   if (!rc) rc = flux(2, in2, U, fd);
+  if (!rc) rc = launch_emf(g, in2, d->sw, d->e, d->stream, kt, fp32, fp32);
   if (!rc && sig) rc = launch_vel_slopes(g, in2, d->sw, d->stream);
   if (!rc && sig) rc = launch_sig_emf(g, in2, d->sw, d->sig, d->stream);
-  if (!rc) rc = launch_emf(g, in2, d->sw, d->e, d->stream, kt, fp32, fp32);
   if (!rc) rc = launch_ct_c2p(g, 2, d->e, fB, fA, oC, U, vn, V, d->flag, d->sc, d->stream, kt, false, ends);
   if (rc) return fail(PGPU_EDEVICE, "stage launch failed: %s", hipGetErrorString((hipError_t)rc));
   // the step's faces are in bC: rotate so that bA is the state again

@@ -85,6 +85,44 @@ def test_signature_leaves_the_step_alone_and_is_deterministic(native):
     assert st_sig == sa
 
 
+# what the signature's kernels store for themselves is not what the step reads:
+# another EMF average or the FP32 flux chosen while it is on
+@pytest.mark.parametrize("emf", ["arithmetic", "uct0", "uct_contact", "uct_hll"])
+def test_signature_leaves_other_averages_alone(native, oracle_lib, emf):
+    from conftest import assert_states_equal
+    from pluto_amd import problems as P
+    _say("case: branch signature on, EMF average %s, random 20^3, 3 steps" % emf)
+    st = P.random_mhd_3d(20, seed=13)
+    dom = native.Domain.from_state(st)
+    dom.set_dt(1e-3, fixed=True)
+    dom.set_branch_signature(True)
+    dom.set_emf_average(emf)
+    dom.run(3)
+    out = dom.get_state(st)
+    dom.close()
+    ref = st.copy()
+    for _ in range(3):
+        oracle_lib.rk2_step(ref, 1e-3, emf=emf)
+    assert_states_equal(out, ref, emf)
+
+
+def test_signature_leaves_fp32_flux_alone(native):
+    from conftest import assert_states_equal
+    from pluto_amd import problems as P
+    st = P.random_mhd_3d(20, seed=13)
+    out = []
+    for sig in (False, True):
+        dom = native.Domain.from_state(st)
+        dom.set_dt(1e-3, fixed=True)
+        if sig:
+            dom.set_branch_signature(True)
+        native.check(native.lib().pgpu_set_precision(dom.h, native.PGPU_PREC_FP32_FLUX))
+        dom.run(3)
+        out.append(dom.get_state(st))
+        dom.close()
+    assert_states_equal(out[0], out[1], "FP32 flux")
+
+
 def test_signature_refuses_what_it_does_not_cover(native):
     from pluto_amd import problems as P
     st = P.random_mhd_3d(16, seed=1)
