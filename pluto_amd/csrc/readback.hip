@@ -69,7 +69,7 @@ int readback(Readback& rb, const ReadSrc& src, double* const* dst, hipStream_t s
 {
   constexpr int NB = Readback::NB;
   const long ni = (long)src.n[0] * src.n[1] * src.n[2], total = ni * src.na;
-  if (total <= 0) return 0;
+  if (total <= 0) return (int)hipStreamSynchronize(s);   // (no array asked for: a wait)
   // (the caller's current device may be another)
   struct OnDevice {
     int was = -1;

@@ -122,3 +122,30 @@ def test_readback(shape, bounded):
         ctypes.POINTER(ctypes.c_double)), None))
     assert np.array_equal(one, st.by)
     dom.close()
+
+
+# a read waits for the steps queued before it, also one that asks for no array
+def test_empty_read_waits():
+    import time
+
+    from pluto_amd import native
+    L = native.lib()
+    st = box_state((256, 256, 256))
+    dom = native.Domain.from_state(st)
+    bat = native.Batch([256])
+    bat.set_patch(0, st)
+    bat.set_dt(1e-4)
+    dom.set_dt(1e-4, fixed=True)
+    for obj, read in ((dom, lambda: L.pgpu_get_state(dom.h, None, None, None, None)),
+                      (bat, lambda: L.pgpu_batch_get_patch(bat.h, 0, None, None, None, None))):
+        obj.run(2)
+        obj.sync()
+        t0 = time.perf_counter()
+        obj.run(60)   # 6 ms each
+        native.check(read())
+        t1 = time.perf_counter()
+        obj.sync()
+        t2 = time.perf_counter()
+        print("run and empty read %.3f s, then the wait %.4f s" % (t1 - t0, t2 - t1), flush=True)
+        assert t2 - t1 < 0.1 * (t1 - t0)
+        obj.close()
