@@ -12,7 +12,9 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstring>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -98,35 +100,27 @@ int readback(Readback& rb, const ReadSrc& src, double* const* dst, hipStream_t s
   };
 
   // chunk c is in its buffer when ready > c; left: threads still copying it
-  std::atomic<long> ready{0};
-  std::atomic<bool> stop{false};
+  std::mutex m;
+  std::condition_variable more;
+  long ready = 0;
+  bool stop = false;
+  int nw = 0;
   std::atomic<int> left[NB];
   for (auto& l : left) l.store(0);
-  std::atomic<int> nworkers{-1};   // (set before the first chunk is ready)
   auto work = [&](int w) {
     for (long c = 0; c < nch; c++) {
-      while (ready.load(std::memory_order_acquire) <= c) {
-        if (stop.load()) return;
-        std::this_thread::yield();
+      {
+        std::unique_lock<std::mutex> lk(m);
+        more.wait(lk, [&] { return ready > c || stop; });
+        if (ready <= c) return;
       }
-      const int nw = nworkers.load();
       const long e0 = c * ch, len = std::min(ch, total - e0);
       const long b = len * w / nw, e = len * (w + 1) / nw;
       copy_out(rb.h[c % NB] + b, e0 + b, e0 + e);
       left[c % NB].fetch_sub(1, std::memory_order_release);
     }
   };
-  // a thread copies about 10 GB/s and starts in about 20 us: from two chunks
-  // on, up to eight
   std::vector<std::thread> th;
-  const int want = nch < 2 ? 0 : (int)std::min(8u, std::max(1u, std::thread::hardware_concurrency() / 2));
-  try {
-    th.reserve(want);
-    for (int w = 0; w < want; w++) th.emplace_back(work, w);
-  } catch (...) {   // fewer threads, or none: this one copies
-  }
-  const int nw = (int)th.size();
-  nworkers.store(nw);
 
   hipError_t err = hipSuccess;
   long issued = 0, got = 0;
@@ -134,7 +128,6 @@ int readback(Readback& rb, const ReadSrc& src, double* const* dst, hipStream_t s
     while (issued < nch && issued - got < NB && left[issued % NB].load(std::memory_order_acquire) == 0) {
       const long e0 = issued * ch, len = std::min(ch, total - e0);
       const long nwg = (len + 1023) / 1024;
-      left[issued % NB].store(nw);
       hipLaunchKernelGGL(k_gather_cells, dim3((unsigned)nwg), dim3(256), 0, s, src, e0, len, rb.h[issued % NB]);
       err = hipGetLastError();
       if (err == hipSuccess) err = hipEventRecord(rb.ev[issued % NB], s);
@@ -148,16 +141,36 @@ int readback(Readback& rb, const ReadSrc& src, double* const* dst, hipStream_t s
     }
     err = hipEventSynchronize(rb.ev[got % NB]);
     if (err != hipSuccess) break;
+    if (got == 0 && nch > 1) {
+      // a thread copies about 10 GB/s and starts in about 20 us: from two chunks
+      // on, up to eight, started only now that there is something to copy (the
+      // stream may hold a whole run of steps before the first chunk)
+      const int want = (int)std::min(8u, std::max(1u, std::thread::hardware_concurrency() / 2));
+      try {
+        th.reserve(want);
+        for (int w = 0; w < want; w++) th.emplace_back(work, w);
+      } catch (...) {   // fewer threads, or none: this one copies
+      }
+      nw = (int)th.size();   // (read after the first chunk is published)
+    }
     if (nw == 0) {
       const long e0 = got * ch;
       copy_out(rb.h[got % NB], e0, std::min(e0 + ch, total));
-      left[got % NB].store(0);
     }
-    ready.store(++got, std::memory_order_release);
+    left[got % NB].store(nw);
+    {
+      std::lock_guard<std::mutex> lk(m);
+      ready = ++got;
+    }
+    more.notify_all();
   }
   // (only a failure stops the threads: after the last chunk they still copy)
   if (err != hipSuccess) {
-    stop.store(true);
+    {
+      std::lock_guard<std::mutex> lk(m);
+      stop = true;
+    }
+    more.notify_all();
     (void)hipStreamSynchronize(s);   // nothing writes the buffers any more
   }
   for (auto& x : th) x.join();

@@ -149,3 +149,28 @@ def test_empty_read_waits():
         print("run and empty read %.3f s, then the wait %.4f s" % (t1 - t0, t2 - t1), flush=True)
         assert t2 - t1 < 0.1 * (t1 - t0)
         obj.close()
+
+
+# while a read waits for the steps queued before it, the host's other processors
+# are left alone (the threads that copy out start when there is something to copy)
+def test_read_waits_idle():
+    import ctypes
+    import resource
+    import time
+
+    from pluto_amd import native
+    st = box_state((256, 256, 256))
+    dom = native.Domain.from_state(st)
+    dom.set_dt(1e-4, fixed=True)
+    out = st.copy()
+    ptrs = [a.ctypes.data_as(ctypes.POINTER(ctypes.c_double)) for a in (out.bx, out.by, out.bz)]
+    native.check(native.lib().pgpu_get_state(dom.h, None, *ptrs))   # (first allocations)
+    dom.run(60)   # 6 ms each
+    t0, c0 = time.perf_counter(), resource.getrusage(resource.RUSAGE_SELF)
+    native.check(native.lib().pgpu_get_state(dom.h, None, *ptrs))
+    t1, c1 = time.perf_counter(), resource.getrusage(resource.RUSAGE_SELF)
+    dom.close()
+    wall, cpu = t1 - t0, c1.ru_utime + c1.ru_stime - c0.ru_utime - c0.ru_stime
+    print("read %.3f s, %.3f s of processor time" % (wall, cpu), flush=True)
+    assert wall > 0.1
+    assert cpu < 2.0 * wall   # one waiting thread, and the copies' 10 ms of eight
