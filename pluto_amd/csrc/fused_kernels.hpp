@@ -104,10 +104,14 @@ inline RowLaunch row_launch(const Geo& g, int real_bytes)
     }
   };
   const int deep = patch_depth(g);
-  // (a workgroup's rows belong to one patch of a stack, which has no windows)
+  // (a workgroup's rows belong to one patch of a stack, which has no windows;
+  // the grid's y, the planes', holds 65535 workgroups: long rows of many planes
+  // take the tiles)
   if (g.pz <= 0)
-    for (int nt = 64; nt <= 256; nt += 64)
-      offer(nt, ((long)g.nz * (g.nx + 4) - 4 + nt - 5) / (nt - 4), 0);
+    for (int nt = 64; nt <= 256; nt += 64) {
+      const long wgs = ((long)g.nz * (g.nx + 4) - 4 + nt - 5) / (nt - 4);
+      if (wgs <= 65535) offer(nt, wgs, 0);
+    }
   for (int r = 1; r * g.nx <= 256 && r <= deep; r++)
     if (g.pz <= 0 || deep % r == 0) offer((r * g.nx + 63) / 64 * 64, ((long)g.nz + r - 1) / r, r);
   if (real_bytes == 8 && g.pz <= 0 && flux_xy_seg() <= 0) {
