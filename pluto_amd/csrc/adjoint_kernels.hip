@@ -979,10 +979,8 @@ static int adj_forward(pgpu_domain* d, const StepTape& T, double* const outB[3])
     fd1.SL[dd] = sw1.d[dd].SL;
     fd2.SR[dd] = sw2.d[dd].SR;
     fd2.SL[dd] = sw2.d[dd].SL;
-    for (int c = 0; c < 3; c++) {
-      fd1.dv[dd][c] = sw1.d[dd].dv[c];
-      fd2.dv[dd][c] = sw2.d[dd].dv[c];
-    }
+    fd1.mf[dd] = sw1.d[dd].dv[0];
+    fd2.mf[dd] = sw2.d[dd].dv[0];
   }
   int rc = launch_flux_fused(g, 1, false, in1, U, fd1, d->cdt, d->sc, s, nullptr);
   if (!rc) rc = launch_vel_slopes(g, in1, sw1, s);

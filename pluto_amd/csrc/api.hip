@@ -759,7 +759,7 @@ static int enqueue_step_fused(pgpu_domain* d)
   for (int a = 0; a < 3; a++) {
     fd.SL[a] = d->sw.d[a].SL;
     fd.SR[a] = d->sw.d[a].SR;
-    for (int c = 0; c < 3; c++) fd.dv[a][c] = d->sw.d[a].dv[c];
+    fd.mf[a] = d->sw.d[a].dv[0];
   }
   FaceIn fA, fB;
   FaceOut oB, oC;
@@ -883,7 +883,7 @@ extern "C" int pgpu_set_emf_tiling(int bx, int by, int kz)
 
 extern "C" int pgpu_set_emf_kernel(int kind, int kz)
 {
-  if (set_emf_kernel(kind, kz)) return fail(PGPU_EINVAL, "EMF kernel %d (kz %d): kind 0, 1 or 2, kz >= 0", kind, kz);
+  if (set_emf_kernel(kind, kz)) return fail(PGPU_EINVAL, "EMF kernel %d (kz %d): kind 0 to 3, kz >= 0", kind, kz);
   return PGPU_OK;
 }
 

@@ -393,8 +393,10 @@ __global__ void k_batch_copy_faces(const double* c0, const double* c1, const dou
 
 using namespace pgpu;
 
-// an edge the stacked mode takes: the row kernel's and the LDS EMF's
-// conditions (even, 4 to 256 cells)
+// an edge the stacked mode takes: even (every stack then starts an even number
+// of cells into its arrays, as the LDS EMF's 16-byte copies like it), 4 to 256
+// cells (whole rows in a workgroup of the row kernel).  The kernels themselves
+// take odd edges too, which run on the persistent kernel
 static bool stack_edge(int n) { return n >= 4 && n <= 256 && n % 2 == 0; }
 
 struct pgpu_batch {
@@ -486,7 +488,8 @@ static int enqueue_stack(pgpu_batch* b, const pgpu_batch::Stack& st, int stage, 
     sw.d[a].SL = fd.SL[a] = A.sw[a][6] + o;
     sw.d[a].SR = fd.SR[a] = A.sw[a][7] + o;
     sw.d[a].cm = A.sw[a][8] + o;
-    for (int k = 0; k < 3; k++) sw.d[a].dv[k] = fd.dv[a][k] = A.sw[a][9 + k] + o;
+    for (int k = 0; k < 3; k++) sw.d[a].dv[k] = A.sw[a][9 + k] + o;
+    fd.mf[a] = sw.d[a].dv[0];
   }
   double* cdt = A.sw[0][0] + o;   // (the flux arrays of the modular sweeps are free here)
   EdgeOut e;

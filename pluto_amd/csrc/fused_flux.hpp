@@ -185,7 +185,7 @@ k_flux_xy(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScalars* sc
       if constexpr (E == FACE_BFLUX) {
         fd.SL[0][cf] = -r.f[BX2];   // ezi, eyi (ct_emf.c:131-133)
         fd.SR[0][cf] = r.f[BX3];
-        fd.dv[0][0][cf] = r.f[RHO];
+        fd.mf[0][cf] = r.f[RHO];
       } else {
         face_store(fd.SL[0], cf, max_ge(R(0), -r.SL));
         face_store(fd.SR[0], cf, max_ge(R(0), r.SR));
@@ -223,7 +223,7 @@ k_flux_xy(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, DevScalars* sc
       if constexpr (E == FACE_BFLUX) {
         fd.SL[1][cf] = r.f[BX1];    // ezj, exj (ct_emf.c:153-155)
         fd.SR[1][cf] = -r.f[BX3];
-        fd.dv[1][0][cf] = r.f[RHO];
+        fd.mf[1][cf] = r.f[RHO];
       } else {
         face_store(fd.SL[1], cf, max_ge(R(0), -r.SL));
         face_store(fd.SR[1], cf, max_ge(R(0), r.SR));
@@ -722,7 +722,7 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
       if constexpr (E == FACE_BFLUX) {
         at_byte(fd.SL[0], cf) = xe[0];
         at_byte(fd.SR[0], cf) = xe[1];
-        at_byte(fd.dv[0][0], cf) = xe[2];
+        at_byte(fd.mf[0], cf) = xe[2];
       } else {
         fstore(fd.SL[0], cf, xsl);
         fstore(fd.SR[0], cf, xsr);
@@ -761,7 +761,7 @@ k_flux_xy_rows(Geo g, StageIn in, Cons U, FaceData fd, double* cdt_xy, int seg, 
         if constexpr (E == FACE_BFLUX) {
           at_byte(fd.SL[1], c) = r.f[BX1];    // ezj, exj (ct_emf.c:153-155)
           at_byte(fd.SR[1], c) = -r.f[BX3];
-          at_byte(fd.dv[1][0], c) = r.f[RHO];
+          at_byte(fd.mf[1], c) = r.f[RHO];
         } else {
           fstore(fd.SL[1], c, max_ge(R(0), -r.SL));
           fstore(fd.SR[1], c, max_ge(R(0), r.SR));
@@ -936,7 +936,7 @@ k_flux_z(Geo g, StageIn in, Cons U, FaceData fd, const double* cdt_xy, int seg, 
       if constexpr (E == FACE_BFLUX) {
         at_byte(fd.SL[2], c) = -r.f[BX1];    // eyk, exk (ct_emf.c:175-176)
         at_byte(fd.SR[2], c) = r.f[BX2];
-        at_byte(fd.dv[2][0], c) = r.f[RHO];
+        at_byte(fd.mf[2], c) = r.f[RHO];
       } else {
         fstore(fd.SL[2], c, max_ge(R(0), -r.SL));
         fstore(fd.SR[2], c, max_ge(R(0), r.SR));

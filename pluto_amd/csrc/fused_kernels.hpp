@@ -35,13 +35,13 @@ inline int march_len(int most, int line, W waves)
   return best;
 }
 
-// Per-face UCT_HLL speeds written by the flux kernels for the EMF kernel
-// (same arrays as SweepOut's; dv[direction][0]: the mass flux of the other
-// EMF averages).
+// Per-face UCT_HLL speeds written by the flux kernels for the EMF kernel; for
+// the other EMF averages the face EMFs and the mass flux mf (same arrays as
+// SweepOut's: SL, SR, dv[0]).
 struct FaceData {
   double* SL[3];
   double* SR[3];
-  double* dv[3][3];
+  double* mf[3];
 };
 
 // fp32_flux: PLM and HLLD in FP32 (states rounded from FP64 on load); the

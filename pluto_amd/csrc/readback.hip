@@ -4,9 +4,11 @@
 // buffers over the link, a ring of four buffers ahead of the host threads
 // that copy them out.  hipMemcpy to pageable memory moved 16 GB/s, one copy
 // and one wait per array, and a ghosted box's arrays came whole and were cut
-// on the host by one thread: 128^3 read back from a periodic box 11.3 -> 3.9
-// ms (48 GB/s; the link 57), from a bounded one 20.7 -> 3.9 ms, 32^3 0.27 ->
-// 0.15 and 0.33 -> 0.15 ms, 96 patches of edges 16 to 64 one by one 47 -> 26.
+// on the host by one thread: 128^3 read back from a periodic box 10.4 -> 3.7
+// ms (50 GB/s; the link 57), from a bounded one 20.0 -> 3.7 ms, 32^3 0.24 ->
+// 0.13 and 0.31 -> 0.13 ms, 96 patches of edges 16 to 64 one by one 47 -> 26.
+// A box's first read also pins its buffers: 128^3 10.5 -> 4.1 ms, 32^3 0.26 ->
+// 0.19 (a process's very first ones, on new host memory, about 1 ms more).
 
 #include "readback.hpp"
 
