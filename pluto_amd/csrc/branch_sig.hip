@@ -68,7 +68,7 @@ __device__ __forceinline__ void sig_dir(const Geo& g, const Cell& p, const Stage
   for (int nv = 0; nv < NV; nv++) {
     const double* a = in.V[nv];
     const double v_m1 = a[cm1], v_0 = a[p.c], v_p1 = a[cp1], v_p2 = a[cp2];
-    const double s0 = mc_slope(v_m1, v_0, v_p1, rec);   // this cell's cases
+    const double s0 = mc_slope_cases(v_m1, v_0, v_p1, rec);   // this cell's cases
     const double s1 = mc_slope(v_0, v_p1, v_p2);        // the next cell's, recorded there
     vL[nv] = v_0 + s0 * 0.5;
     vR[nv] = v_p1 - s1 * 0.5;

@@ -73,12 +73,14 @@ int flux_xy_seg();
 // segment's start), 512 workgroups of three or four waves (three: 0.8 of
 // the time) run at once, half as many in 0.65 of the time; whole rows go in
 // rounds, the windows' workgroups drift apart and end ragged (f + 0.4).
-// Measured at 256^3 1255 us (16 rows: 1294), 128^3 as two rows a workgroup
-// 176 (one row: 180, and 299 against 206 at 32 rows), 64^3 36 (one row a
-// workgroup: 47), 16 x 256^2 91 (windows of one row: 196), 133^3 windows
-// 8 rows 278 (32: 304), 261 x 256^2 16 rows 1345 (8: 1434), 384 x 288 x 320
-// 2790 (tiles: 3792).  (Both kernels wrote the velocity slopes then; without
-// them every figure is about 7% less, 256^3 1180 and 384 x 288 x 320 2570.)
+// The units were measured when both kernels still wrote the velocity slopes;
+// the choice needs their ratios only.  Present times in us, the choice and
+// another: 256^3 32 rows 1153 (16: 1174), 128^3 as two rows a workgroup, 16
+// rows, 161 (8: 167, 32: 189), 64^3 2 rows 34 (1: 39, tiles 49), 16 x 256^2 8
+// rows 85 (16: 96, tiles 110), 133^3 windows 209 (8 rows, the best, 199; 32:
+// 288, tiles 253), 261 x 256^2 16 rows 1217 (8: 1286, tiles 1648), 96^3 98 (4
+// rows, the best, 91; tiles 113); of the sizes near the tiles' line, 48^3 24.6
+// (tiles 25.0), a 512^2 plane 34.5 by tiles (1 to 4 rows: 43 to 50), 32^3 16.7 (tiles 19.5).
 struct RowLaunch {
   int nt = 0, wgs = 0, rows = 0, seg = 0;
 };

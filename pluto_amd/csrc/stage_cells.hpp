@@ -66,8 +66,8 @@ __device__ __forceinline__ double sweep_cell(const Geo& g, const Cell& p, const 
   for (int nv = 0; nv < NV; nv++) {
     const double* a = in.V[nv];
     const double v_m1 = a[cm1], v_0 = a[p.c], v_p1 = a[cp1], v_p2 = a[cp2];
-    const double s0 = mc_slope(v_m1, v_0, v_p1, own);
-    const double s1 = mc_slope(v_0, v_p1, v_p2, next);
+    const double s0 = mc_slope_cases(v_m1, v_0, v_p1, own);
+    const double s1 = mc_slope_cases(v_0, v_p1, v_p2, next);
     const double vp0 = v_0 + s0 * 0.5;   // cell q, right face
     const double vm0 = v_0 - s0 * 0.5;   // cell q, left face
     const double vm1 = v_p1 - s1 * 0.5;  // cell q+1, left face
