@@ -499,11 +499,23 @@ void get_emf_tiling(int* bx, int* by, int* kz)
   *kz = g_emf_kz;
 }
 
+// Whether the register kernels beat the LDS one where the sweeps have stored the
+// velocity slopes (modular pipeline): on small boxes, but for narrow ones that
+// an LDS tile holds whole.  us a launch, register and LDS: 33^3 11.5 and 14.1,
+// 64^3 18.4 and 22.1, 300 x 3 x 300 22.9 and 49.4, 256^2 6.8 and 8.1, 3 x 3 x
+// 2000 29.5 and 43.2; 100^3 84.7 and 75.3, 7 x 7 x 500 23.1 and 14.6, 3 x 300
+// x 300 292.8 and 155.5, 1000^2 34.1 and 26.7.
+static bool emf_by_registers(const Geo& g)
+{
+  return g.n <= 300000 && (g.nx >= 16 || g.nx * g.ny < 16);
+}
+
 // f32_faces: face speeds and velocity slopes stored as float (FP32 flux);
-// f32_state: the velocities of the stage input too (FP32 flux, stage 2)
+// f32_state: the velocities of the stage input too (FP32 flux, stage 2);
+// slopes: the velocity slopes are in sw already
 static bool enqueue_emf(const Geo& g, const StageIn& in, const Sweeps& sw, const EdgeOut& e,
                         hipStream_t s, KernelTimer* kt, bool f32_faces = false,
-                        bool f32_state = false)
+                        bool f32_state = false, bool slopes = false)
 {
   if (g.pz > 0 && g.emf_avg != EMF_UCT_HLL) return false;
   if (g.emf_avg == EMF_ARITHMETIC) {
@@ -516,12 +528,12 @@ static bool enqueue_emf(const Geo& g, const StageIn& in, const Sweeps& sw, const
     if (kt) kt->begin(KT_EMF, s);
     launch_emf_faces<EMF_UCT_CONTACT>(g, in, sw, e, s);
     if (kt) kt->end(KT_EMF, s);
-  } else if ((g_emf_kernel || g.pz > 0 || g.dims != 3) &&
+  } else if ((g_emf_kernel || g.pz > 0 || g.dims != 3) && !(slopes && emf_by_registers(g)) &&
              launch_emf_lds(g, in, sw, e, s, g_emf_kernel ? g_emf_kernel : 3, g_emf_lds_kz, kt,
                             f32_state ? 2 : (f32_faces ? 1 : 0))) {
     // LDS-staged z-march (the only EMF kernel for a stack of patches)
   } else if (g.pz > 0 ||
-             launch_vel_slopes(g, in, sw, s, f32_state ? 2 : (f32_faces ? 1 : 0)) != 0) {
+             (!slopes && launch_vel_slopes(g, in, sw, s, f32_state ? 2 : (f32_faces ? 1 : 0)) != 0)) {
     return false;
   } else if (g.dims == 3 && (unsigned long long)g.n * 8ull < (1ull << 32)) {
     const dim3 b(g_emf_bx, g_emf_by, 1);
@@ -556,7 +568,7 @@ int launch_emf_ct(const Geo& g, bool blend, const StageIn& in, const Sweeps& sw,
   // the modular sweeps store the UCT_HLL face data only
   if (g.emf_avg != EMF_UCT_HLL) return (int)hipErrorInvalidValue;
   const dim3 gr = grid_of(g);
-  enqueue_emf(g, in, sw, e, s, kt);
+  enqueue_emf(g, in, sw, e, s, kt, false, false, true);
   if (!blend) PGPU_TIMED(KT_CT, k_ct<1>, gr, kBlock, 0, s, g, e, bin, b0, bout, sc);
   else PGPU_TIMED(KT_CT, k_ct<2>, gr, kBlock, 0, s, g, e, bin, b0, bout, sc);
   return (int)hipGetLastError();

@@ -79,9 +79,9 @@ def test_rows(shape, seg):
 # the LDS EMF: tiles cut at the row and plane ends, even rows (16-byte copies)
 # and odd ones (4-byte), boxes narrower than a tile, z segments with a
 # remainder, 2D
-@pytest.mark.parametrize("shape", [(3, 3, 3), (5, 9, 31), (17, 8, 32), (18, 7, 33), (6, 10, 34),
-                                   (33, 17, 66), (1, 3, 3), (1, 9, 32), (1, 25, 67)])
-@pytest.mark.parametrize("kind", [1, 2, 3])
+@pytest.mark.parametrize("kind,shape", [(k, s) for k in (1, 2, 3) for s in (
+    (3, 3, 3), (5, 9, 31), (17, 8, 32), (18, 7, 33), (6, 10, 34), (33, 17, 66))]
+    + [(3, s) for s in ((1, 3, 3), (1, 9, 32), (1, 25, 67))])   # (2D has one kernel)
 def test_emf_tiles(shape, kind):
     from pluto_amd import native
     native.set_emf_kernel(kind)
@@ -99,6 +99,21 @@ def test_emf_tiles(shape, kind):
 @pytest.mark.parametrize("emf", ["uct0", "uct_contact", "arithmetic"])
 def test_emf_faces(shape, emf):
     check(shape, dims=2 if shape[0] == 1 else 3, emf=emf)
+
+
+# the modular pipeline's EMF: register kernels on small boxes, the LDS one on
+# larger and on narrow ones (either side of 300000 cells, 16-cell rows, 16-cell
+# planes), 2D too
+@pytest.mark.parametrize("shape", [(3, 3, 3), (20, 5, 3), (20, 6, 3), (9, 20, 15), (9, 20, 16), (64, 64, 73),
+                                   (65, 65, 72), (1, 4, 3), (1, 20, 16), (1, 547, 548), (1, 549, 550)])
+@pytest.mark.parametrize("kind", [0, 3])
+def test_modular_emf(shape, kind):
+    from pluto_amd import native
+    native.set_emf_kernel(kind)
+    try:
+        check(shape, dims=2 if shape[0] == 1 else 3, pipeline=native.PIPELINE_MODULAR)
+    finally:
+        native.set_emf_kernel()
 
 
 # read-back: less than one staging buffer (2^19 values), just over one and
