@@ -5,7 +5,9 @@ comes from the device-side CFL reduction over PLUTO's ranges.  Against
 PLUTO's own main loop with the same [Boundary] block (oracle/_ref/pluto3d,
 the state loader setting the face below the first cell as the image of the
 last face, as the bounded box does), bit for bit: states, dt and Mach per
-dumped step.  div.B stays at round-off in the interior cells.
+dumped step.  div.B stays at round-off in the interior cells.  Periodic axes,
+alone and beside outflow ones, also against the oracle, with lower faces that
+differ from the last ones.
 """
 import numpy as np
 import pytest
