@@ -207,7 +207,8 @@ int  pgpu_set_emf_kernel (int kind, int kz);
    or of windows of them (rows wider than 256 cells among others), marching
    up y segments of seg rows (0: by size, 32 at most), each cell
    reconstructed once per direction, on boxes with fields under 4 GiB; with
-   seg 0 small FP64 boxes still take the tiles where those are faster. */
+   seg 0 small FP64 boxes and narrow FP32 planes still take the tiles where
+   those are faster, and rows wider than 256 in too many planes for the grid. */
 int  pgpu_set_flux_kernel (int kind, int seg);
 
 /* Host <-> device state copies (synchronous).  prim is [8][nz][ny][nx];

@@ -123,6 +123,15 @@ inline RowLaunch row_launch(const Geo& g, int real_bytes)
     const double us = f <= 1.0 ? 12.0 + 14.0 * f : 3.0 + 17.0 * (f <= 4.0 ? (double)(long)(f + 0.9999) : f + 0.3);
     if (us < 5.0 + 9.6 * cost) best.nt = 0;
   }
+  if (real_bytes == 4 && g.pz <= 0 && flux_xy_seg() <= 0 && best.nt == 64) {
+    // FP32 rows too short and in too few planes for more than one wave a
+    // workgroup: tiles where there are many such rows and few tiles.  us, tiles
+    // and rows: planes of 3 x 2000 14.8 and 24.0, 16 x 800 12.3 and 20.2, 60 x 5000
+    // 32.7 and 35.0, 9 x 1200 x 3 16.7 and 20.4; 3 x 1500 x 15 44.7 and 23.2,
+    // 3 x 500 16.0 and 15.0, 64^2 13.4 and 11.2
+    const double us = 12.0 + 0.013 * (double)((g.nx + 31) / 32) * ((g.ny + 7) / 8) * g.nz;
+    if ((long)best.wgs * g.ny > 700 && us < 5.0 + 7.0 * cost) best.nt = 0;
+  }
   return best;
 }
 // the FP32-flux launches (fused_f32.hip, compiled with FMA contraction)
